@@ -230,8 +230,9 @@ sdhip_status sdhip_conv2d(const sdhip_tensor *kernel, const sdhip_tensor *input,
  * and 160, the keys and values split into FP16 parts, tile by tile, and,
  * where the queries alone leave the device's CUs idle and the keys are split
  * across blocks, each split's maximum, sum and output; the same for heads of
- * more than 256 dimensions whose keys are split across blocks; 0 for the
- * other forms.  A buffer short of
+ * more than 256 dimensions whose keys are split across blocks, and for heads
+ * of 388 .. 512 over many positions the queries, keys and values split into
+ * FP16 parts; 0 for the other forms.  A buffer short of
  * sdhip_attention_work_size is SDHIP_ERROR.  Replaces attention_supported /
  * attention_work_size / attention_compute (ops.h:51-56). */
 int sdhip_attention_supported(const sdhip_tensor *q, const sdhip_tensor *k, const sdhip_tensor *v,

@@ -70,4 +70,12 @@ size_t attention_lds_bytes(int64_t d, int64_t dv);
 size_t attention_work_bytes(const AttentionArgs &a);
 hipError_t launch_attention(AttentionArgs a, void *work, hipStream_t stream);
 
+// Heads of 388 .. 512 dimensions over many positions (attention512.hip): the
+// shapes it takes, those with the alignment it asks for too, its work buffer
+// and its launch.
+bool attention512_shape(const AttentionArgs &a);
+bool attention512_taken(const AttentionArgs &a);
+size_t attention512_work_bytes(const AttentionArgs &a);
+hipError_t launch_attention512(AttentionArgs a, void *work, hipStream_t stream);
+
 }  // namespace sdhip

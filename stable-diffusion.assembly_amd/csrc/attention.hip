@@ -431,7 +431,8 @@ __global__ __launch_bounds__(256) void attention_wide_kernel(AttentionArgs a, in
 }
 
 // Heads of up to 512 dimensions (more than 384) with single-precision keys
-// and values (the VAE's middle block, 512): the wide form's products, softmax and sums, in the same
+// and values, where attention512.hip does not take them (fewer positions,
+// rows not 16-byte aligned, or attention_fp32=1): the wide form's products, softmax and sums, in the same
 // order -- bit for bit its output -- with each wave's 16 queries held in
 // registers for the whole split (lane (lr, lg) holds dimensions 4 j + lg of
 // query lr: operand B of step j) and a block's 32 keys and their values
@@ -1906,7 +1907,11 @@ size_t attention_work_bytes(const AttentionArgs &a) {
     if (split_form(a)) return split_form_work(a);
     if (wide_form(a)) {
         const WideSplits w = wide_splits(a);
-        return w.splits > 1 ? static_cast<size_t>(a.b * a.h * w.splits * a.lq * (12 + 4 * a.dv)) : 0;
+        const size_t wide = w.splits > 1 ? static_cast<size_t>(a.b * a.h * w.splits * a.lq * (12 + 4 * a.dv)) : 0;
+        // Either form's: which of the two a call takes depends on its
+        // operands' alignment, which the query of the size may not know.
+        const size_t split = attention512_shape(a) ? attention512_work_bytes(a) : 0;
+        return split > wide ? split : wide;
     }
     return 0;
 }
@@ -1914,6 +1919,7 @@ size_t attention_work_bytes(const AttentionArgs &a) {
 hipError_t launch_attention(AttentionArgs a, void *work, hipStream_t stream) {
     if (a.lq == 0 || a.h == 0 || a.b == 0) return hipSuccess;  // no output
     if (split_form(a)) return launch_split_form(a, work, stream);
+    if (attention512_taken(a)) return launch_attention512(a, work, stream);
     if (fast_form(a) && tuning().attention_generic == 0 && !a.bf16) return launch_fast_form(a, stream);
     a.dp = static_cast<int>(round_up(a.d, 4));
     a.ldq = a.dp + 1;

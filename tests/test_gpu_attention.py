@@ -273,3 +273,42 @@ def test_attention_key_splits(gpu, c):
     print(f"attention key splits {c}: {err:.3g}")
     assert np.isfinite(y).all()
     assert err <= BOUND
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [(512, 1024, 1024, 1, 1, 1), (512, 1000, 1027, 1, 1, 1), (388, 1, 16385, 1, 1, 1),
+                               (500, 257, 1025, 4, 2, 1), (512, 2049, 545, 1, 1, 2)],
+                         ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("spread", [0, 12])
+def test_attention512(gpu, c, spread):
+    """Heads of 388 .. 512 dimensions in split FP16: ragged tiles of queries
+    and keys, an odd count of key tiles, one query, heads sharing keys, the
+    keys in one split and several; with `spread`, values whose magnitude
+    moves by up to 2^(+-spread) from one run of 32 keys to the next, so that
+    the outputs' exponent moves, and keys and queries of 2^+-spread whose
+    products stay.  Within the bound of float64, and no further from it than
+    the products of single precision (attention_fp32=1), the sums' orders
+    aside."""
+    d, lq, lk, h, hk, b = c
+    r = rng(d + lq + lk + spread)
+    q, k, v = (r.standard_normal(s).astype(np.float32) for s in ((b, lq, h, d), (b, lk, hk, d), (b, lk, hk, d)))
+    if spread:
+        v *= np.exp2(r.integers(-spread, spread + 1, (lk + 31) // 32)).repeat(32)[:lk, None, None].astype(np.float32)
+        q *= np.float32(2.0 ** spread)
+        k *= np.float32(2.0 ** -spread)
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(d)))
+    exact, mag = orc.exact_attention(q, k, v, scale)
+    views = [dev(t, gpu).permute(0, 2, 1, 3) for t in (q, k, v)]
+    errors = {}
+    for tuning in ("", "attention_fp32=1"):
+        y = unwritten((b, lq, h, d), gpu)
+        sdhip.set_tuning(tuning)
+        try:
+            sdhip.attention(*views, y, scale)
+        finally:
+            sdhip.set_tuning("")
+        torch.cuda.synchronize()
+        errors[tuning] = orc.metric(y.cpu().numpy(), exact, mag)
+    print(f"attention {c} spread {spread}: {errors}")
+    assert errors[""] <= BOUND
+    assert errors[""] <= 1.5 * errors["attention_fp32=1"] + 1e-7
