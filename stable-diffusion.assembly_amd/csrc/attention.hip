@@ -930,9 +930,6 @@ struct Split {
     static constexpr int kRecord = (2 * kHalves + 1023) / 1024 * 1024;  // bytes of a tile, whole KB
     static constexpr int kCopies = kRecord / 1024;                      // 1 KB copies of a tile
     static constexpr int kPerWave = (kCopies + 3) / 4;
-    // The LDS buffers of the form that splits the keys and values itself
-    // (LOCAL): as large as both planes in full, for its staging.
-    static constexpr int kLocalBuffer = (4 * (kPlaneK + kPlaneV) + 1023) / 1024 * 1024;
     static_assert(D % 8 == 0 && KB % 32 == 0, "shape");
     static_assert(!kHalfStep || kDp == D + 8, "the keys' low parts fill the last step's padding");
     static_assert((kLdkl / 8) % 2 == 1, "rows of an odd number of 16-byte units");
@@ -1130,6 +1127,126 @@ __device__ __forceinline__ void split_exp(float (&p)[KT][16], float shift, doubl
     if constexpr (SUM) l += part;
 }
 
+// A query, times scale log2(e), as operand B of S^T: the lane of half g holds
+// dimensions 16 st + 8 g .. + 7 at step st, q(st, j, dim) its j-th there.  With
+// kHalfStep the last step's upper half holds h' of the dimension 8 below its
+// own where the others hold l', and zero where they hold h'.
+template <int D, int KB, class Q>
+__device__ __forceinline__ void split_query(Q q, float scale, int g, half8 (&qh)[Split<D, KB>::kSteps],
+                                            half8 (&ql)[Split<D, KB>::kSteps]) {
+    using S = Split<D, KB>;
+    const float qscale = scale * 1.44269504088896341f;
+#pragma unroll
+    for (int st = 0; st < S::kSteps; ++st)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const bool slot = S::kHalfStep && st == S::kSteps - 1 && g == 1;
+            const int dim = 16 * st + 8 * g + j - (slot ? 8 : 0);
+            _Float16 h, l;
+            split_part(dim < D ? (q(st, j, dim) * qscale) * kSplitDown : 0.0f, h, l);
+            qh[st][j] = slot ? static_cast<_Float16>(0.0f) : h;
+            ql[st][j] = slot ? h : l;
+        }
+}
+
+// S^T of a tile from its keys' parts: h h' into sh, h l' + l h' into sx.
+template <int D, int KB>
+__device__ __forceinline__ void score_products(const half8 (&kah)[Split<D, KB>::kSteps][Split<D, KB>::kTiles],
+                                               const half8 (&kal)[Split<D, KB>::kSteps][Split<D, KB>::kTiles],
+                                               const half8 (&qh)[Split<D, KB>::kSteps],
+                                               const half8 (&ql)[Split<D, KB>::kSteps],
+                                               float16v (&sh)[Split<D, KB>::kTiles],
+                                               float16v (&sx)[Split<D, KB>::kTiles]) {
+    using S = Split<D, KB>;
+#pragma unroll
+    for (int u = 0; u < S::kTiles; ++u) {
+        sh[u] = float16v{};
+        sx[u] = float16v{};
+    }
+#pragma unroll
+    for (int st = 0; st < S::kSteps; ++st)
+#pragma unroll
+        for (int u = 0; u < S::kTiles; ++u) {
+            sh[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kah[st][u], qh[st], sh[u], 0, 0, 0);
+            sx[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kah[st][u], ql[st], sx[u], 0, 0, 0);
+            if (!S::kHalfStep || st < S::kSteps - 1)
+                sx[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kal[st][u], qh[st], sx[u], 0, 0, 0);
+        }
+}
+
+// O^T += V^T P^T of a tile, a chunk of 16 keys at a time: the lane's eight
+// exponentials 8 c .. 8 c + 7 of a tile of 32 are its operand B, taken
+// (2^11 times, below 2^15) as two FP16 parts, the second the remainder of the
+// first.  minus_one is -1 where the compiler does not see it: x - h is then
+// one v_fma_mix_f32 rather than a conversion and a subtraction.
+template <int D, int KB>
+__device__ __forceinline__ void value_products(const float (&p)[Split<D, KB>::kTiles][16],
+                                               const half8 (&vah)[Split<D, KB>::kTiles][2][Split<D, KB>::kDvt],
+                                               const half8 (&val)[Split<D, KB>::kTiles][2][Split<D, KB>::kDvt],
+                                               float16v (&oh)[Split<D, KB>::kDvt], float16v (&ol)[Split<D, KB>::kDvt],
+                                               float minus_one) {
+    using S = Split<D, KB>;
+#pragma unroll
+    for (int u = 0; u < S::kTiles; ++u)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            half8 ph, pl;
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                const float x0 = p[u][8 * c + j], x1 = p[u][8 * c + j + 1];
+                const auto h = __builtin_amdgcn_cvt_pkrtz(x0, x1);
+                const auto r = __builtin_amdgcn_cvt_pkrtz(__builtin_fmaf(static_cast<float>(h[0]), minus_one, x0),
+                                                          __builtin_fmaf(static_cast<float>(h[1]), minus_one, x1));
+                ph[j] = h[0];
+                ph[j + 1] = h[1];
+                pl[j] = r[0];
+                pl[j + 1] = r[1];
+            }
+#pragma unroll
+            for (int dt = 0; dt < S::kDvt; ++dt) {
+                oh[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vah[u][c][dt], ph, oh[dt], 0, 0, 0);
+                oh[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vah[u][c][dt], pl, oh[dt], 0, 0, 0);
+                if (!S::kPackV || dt < S::kDvt - 1)  // the packed tile's low parts are rows of vah
+                    ol[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(val[u][c][dt], ph, ol[dt], 0, 0, 0);
+            }
+        }
+}
+
+// The query's sum over its two lanes, or from the rows of ones (the same on
+// both).
+template <int D, int KB>
+__device__ __forceinline__ double sum_of(double l, const float16v (&oh)[Split<D, KB>::kDvt]) {
+    using S = Split<D, KB>;
+    if constexpr (S::kSumRow) return static_cast<double>(oh[S::kDvt - 1][S::kVLast]) * 16.0;
+    return l + __shfl_xor(l, 32, 64);
+}
+
+// The query's output: the lane holds O^T[32 dt + 8 (e / 4) + 4 g + e % 4], and
+// the values' 2^-4 comes back with the reciprocal.  The packed tile's low
+// parts are kVLast rows, kVLast / 2 elements, below its high parts.
+template <int D, int KB>
+__device__ __forceinline__ void store_query(double sum, const float16v (&oh)[Split<D, KB>::kDvt],
+                                            const float16v (&ol)[Split<D, KB>::kDvt], int g, float *out) {
+    using S = Split<D, KB>;
+    const float reciprocal = static_cast<float>(1.0 / sum);
+#pragma unroll
+    for (int dt = 0; dt < S::kDvt; ++dt)
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4) {
+            const int dim = 32 * dt + 8 * e4 + 4 * g;
+            if (dim < D) {
+                float4v r;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int e = 4 * e4 + u;
+                    const float low = S::kPackV && dt == S::kDvt - 1 ? oh[dt][e + S::kVLast / 2] : ol[dt][e];
+                    r[u] = ((oh[dt][e] + low * kPartDown) * 16.0f) * reciprocal;
+                }
+                *reinterpret_cast<float4v *>(out + dim) = r;
+            }
+        }
+}
+
 // Partial results of the split form's key splits: per (b h, split, query)
 // the running maximum, the sum and the unnormalised output.
 struct KeyPartial {
@@ -1138,17 +1255,12 @@ struct KeyPartial {
     float *o;   // [b h][split][lq][dv], 16-byte aligned
 };
 
-template <int D, int KB, int NS, int OCC, bool PIPE, bool LOCAL>
+template <int D, int KB, int NS, int OCC, bool PIPE>
 __global__ __launch_bounds__(256, OCC) void attention_split_kernel(AttentionArgs a, const char *__restrict__ tiles,
                                                                    int64_t splits, int64_t per, KeyPartial part) {
     using S = Split<D, KB>;
     static_assert(NS >= 3 && (NS - 2) * S::kPerWave < 64, "stages");
-    // LDS buffers of kStride bytes: a tile's record, or with LOCAL room for
-    // the staging as well.
-    constexpr int kStride = LOCAL ? S::kLocalBuffer : S::kRecord;
-    static_assert(S::kQueries * D * 4 <= NS * kStride, "the queries' staging fits the ring");
-    static_assert(KB * (D + 4) * 4 <= kStride, "a tile's values fit a buffer as they stand");
-    extern __shared__ __attribute__((aligned(1024))) char sbuf[];  // NS buffers of kStride bytes
+    extern __shared__ __attribute__((aligned(1024))) char sbuf[];  // NS buffers of kRecord bytes
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -1162,19 +1274,10 @@ __global__ __launch_bounds__(256, OCC) void attention_split_kernel(AttentionArgs
     // per) of the head's nk_all and writes partial results for
     // split_combine_kernel; nk is then its own count of tiles.
     // Consecutive blocks of one XCD: the query blocks of a head, which read
-    // the same tiles of keys; with LOCAL (a few keys, every workgroup its own
-    // copies), the heads of a query block instead, whose rows of queries and
-    // of the output lie side by side in memory and share lines.
+    // the same tiles of keys.
     const uint32_t b = xcd_swizzle(blockIdx.x, gridDim.x);
-    uint32_t qb, rest;
-    if constexpr (LOCAL) {
-        const uint32_t heads = static_cast<uint32_t>(a.b * a.h);
-        qb = b / heads;
-        rest = b - qb * heads;
-    } else {
-        qb = b % static_cast<uint32_t>(a.qblocks);
-        rest = b / static_cast<uint32_t>(a.qblocks);
-    }
+    const uint32_t qb = b % static_cast<uint32_t>(a.qblocks);
+    const uint32_t rest = b / static_cast<uint32_t>(a.qblocks);
     const int64_t sp = static_cast<int64_t>(rest % static_cast<uint32_t>(splits));
     const uint32_t bh = rest / static_cast<uint32_t>(splits);
     const int64_t hi = bh % a.h;
@@ -1196,182 +1299,21 @@ __global__ __launch_bounds__(256, OCC) void attention_split_kernel(AttentionArgs
     // bytes: key_splits caps nk), so that each copy's address is the lane's
     // 16 bytes and a scalar offset.
     const __amdgpu_buffer_rsrc_t head_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char *>(head), 0, static_cast<int>(LOCAL ? 0 : nk * S::kRecord), 0x00020000);
+        const_cast<char *>(head), 0, static_cast<int>(nk * S::kRecord), 0x00020000);
     const auto issue = [&](int stage, int64_t t) {
 #pragma unroll
         for (int i = 0; i < S::kPerWave; ++i) {
             int c = swave + 4 * i;
             c = c < S::kCopies ? c : S::kCopies - 1;
             copy_lds_buffer(head_rsrc, lane16, static_cast<uint32_t>(t * S::kRecord + c * 1024),
-                            sbuf + stage * kStride + c * 1024);
+                            sbuf + stage * S::kRecord + c * 1024);
         }
     };
-    // The wave's queries, operand B of S^T: lane (query lr, half g) holds
-    // dimensions 16 st + 8 g .. + 7 at step st; queries past lq read the
-    // last.  With LOCAL (a few tiles of keys, so the queries' loads weigh)
-    // the workgroup's queries go through LDS first, rows of D read as float4
-    // by consecutive threads; otherwise each lane reads its own row.
     half8 qh[S::kSteps], ql[S::kSteps];
-    const float qscale = a.scale * 1.44269504088896341f;  // scale log2(e), folded into the queries
-    // The lane's query (row qp) into its parts.  With kHalfStep the last
-    // step's upper half holds h' of the dimension 8 below its own where the
-    // others hold l', and zero where they hold h'.
-    const auto take_query = [&](const float *qp) {
-#pragma unroll
-        for (int st = 0; st < S::kSteps; ++st)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const bool slot = S::kHalfStep && st == S::kSteps - 1 && g == 1;
-                const int dim = 16 * st + 8 * g + j - (slot ? 8 : 0);
-                _Float16 h, l;
-                split_part(dim < D ? (qp[dim] * qscale) * kSplitDown : 0.0f, h, l);
-                qh[st][j] = slot ? static_cast<_Float16>(0.0f) : h;
-                ql[st][j] = slot ? h : l;
-            }
-    };
-    // LOCAL, where the staging fits: every load of the workgroup -- its
-    // queries, and the keys and values of every tile -- in flight at once,
-    // into registers; then the queries staged in buffers 1 .., the values as
-    // they stand in the spare buffer NS - 1, tile 0's keys split into buffer
-    // 0; past a barrier each lane's query from the staging; past another the
-    // other tiles' keys split, the padding dimensions of the keys cleared and
-    // every tile's values split and transposed from the staging.  One wait for
-    // memory where a tile at a time takes one a tile.
-    constexpr bool kBatch = LOCAL && (NS - 1) * KB * (D + 4) * 4 <= kStride &&
-                            S::kQueries * D * 4 <= (NS - 2) * kStride;
-    if constexpr (kBatch) {
-        constexpr int kQ4 = S::kQueries * (D / 4);  // float4s of the workgroup's queries
-        constexpr int kQPer = (kQ4 + 255) / 256;
-        constexpr int kKV4 = (NS - 1) * KB * (D / 4);  // float4s of the keys (or values) of NS - 1 tiles
-        constexpr int kKVPer = (kKV4 + 255) / 256;
-        const float *qg = a.q + bi * a.qnb3 + hi * a.qnb2;
-        const float *kg = static_cast<const float *>(a.k) + bi * a.knb3 + kh * a.knb2;
-        const float *vg = static_cast<const float *>(a.v) + bi * a.vnb3 + kh * a.vnb2;
-        const int64_t qrow0 = static_cast<int64_t>(qb) * S::kQueries;
-        float4v qv[kQPer], kv[kKVPer], vv[kKVPer];
-#pragma unroll
-        for (int i = 0; i < kQPer; ++i) {
-            const int idx = tid + 256 * i;
-            qv[i] = float4v{};
-            if (idx < kQ4) {
-                const int r = idx / (D / 4), c4 = idx - r * (D / 4);
-                const int64_t row = qrow0 + r < a.lq ? qrow0 + r : a.lq - 1;
-                qv[i] = *reinterpret_cast<const float4v *>(qg + row * a.qnb1 + 4 * c4);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kKVPer; ++i) {
-            const int idx = tid + 256 * i;
-            const int key = idx / (D / 4), c4 = idx - key * (D / 4);
-            kv[i] = float4v{};
-            vv[i] = float4v{};
-            if (idx < kKV4 && key < a.lk) {
-                kv[i] = *reinterpret_cast<const float4v *>(kg + key * a.knb1 + 4 * c4);
-                vv[i] = *reinterpret_cast<const float4v *>(vg + key * a.vnb1 + 4 * c4);
-            }
-        }
-        float *qstage = reinterpret_cast<float *>(sbuf + kStride);              // [kQueries][D]
-        float *vstage = reinterpret_cast<float *>(sbuf + (NS - 1) * kStride);   // [key][D + 4]
-        // Key `key`'s four dimensions 4 c4 .. split into its tile's two planes.
-        const auto put_key = [&](int key, int c4, float4v x) {
-            _Float16 *rec = reinterpret_cast<_Float16 *>(sbuf + (key / KB) * kStride);
-            const int j = key % KB;
-            half4a h, l;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                _Float16 hh, ll;
-                split_part(x[r] * kSplitDown, hh, ll);
-                h[r] = hh;
-                l[r] = ll;
-            }
-            *reinterpret_cast<half4a *>(rec + j * S::kLdk + 4 * c4) = h;
-            if (4 * c4 < S::kLdkl) *reinterpret_cast<half4a *>(rec + S::kPlaneK + j * S::kLdkl + 4 * c4) = l;
-            if (S::kHalfStep && 4 * c4 >= D - 8) *reinterpret_cast<half4a *>(rec + j * S::kLdk + 4 * c4 + 8) = l;
-        };
-#pragma unroll
-        for (int i = 0; i < kQPer; ++i) {
-            const int idx = tid + 256 * i;
-            if (idx < kQ4) {
-                const int r = idx / (D / 4), c4 = idx - r * (D / 4);
-                *reinterpret_cast<float4v *>(qstage + r * D + 4 * c4) = qv[i];
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kKVPer; ++i) {
-            const int idx = tid + 256 * i;
-            const int key = idx / (D / 4), c4 = idx - key * (D / 4);
-            if (idx < kKV4) {
-                *reinterpret_cast<float4v *>(vstage + key * (D + 4) + 4 * c4) = vv[i];
-                if (key < KB) put_key(key, c4, kv[i]);
-            }
-        }
-        __syncthreads();
-        const float *qp = qstage + (wave * 32 + lr) * D;
-        take_query(qp);
-        __syncthreads();  // every wave's queries read before the tiles overwrite their staging
-#pragma unroll
-        for (int i = 0; i < kKVPer; ++i) {
-            const int idx = tid + 256 * i;
-            const int key = idx / (D / 4), c4 = idx - key * (D / 4);
-            if (idx < kKV4 && key >= KB && key < nk * KB) put_key(key, c4, kv[i]);
-        }
-        constexpr int kPad4 = (S::kDp - D) / 4;  // float4s of padding dimensions a key
-        if constexpr (kPad4 > 0 && !S::kHalfStep) {  // with kHalfStep the padding holds low parts
-            for (int idx = tid; idx < nk * KB * kPad4; idx += 256) {
-                const int key = idx / kPad4, c4 = D / 4 + (idx - key * kPad4);
-                put_key(key, c4, float4v{});
-            }
-        }
-        for (int64_t t = 0; t < nk; ++t) {
-            const float *vt = vstage + t * KB * (D + 4);
-            split_values<D, KB>([&](int j, int dim) { return vt[j * (D + 4) + dim]; },
-                                reinterpret_cast<_Float16 *>(sbuf + t * kStride));
-        }
-        __syncthreads();
-    } else {
-        const float *qp;
-        if constexpr (LOCAL) {
-            float *qstage = reinterpret_cast<float *>(sbuf);  // [kQueries][D]
-            const int64_t qrow0 = static_cast<int64_t>(qb) * S::kQueries;
-            for (int idx = tid; idx < S::kQueries * (D / 4); idx += 256) {
-                const int r = idx / (D / 4), c4 = idx - r * (D / 4);
-                int64_t i = qrow0 + r;
-                i = i < a.lq ? i : a.lq - 1;
-                *reinterpret_cast<float4v *>(qstage + r * D + 4 * c4) =
-                    *reinterpret_cast<const float4v *>(a.q + bi * a.qnb3 + hi * a.qnb2 + i * a.qnb1 + 4 * c4);
-            }
-            __syncthreads();
-            qp = qstage + (wave * 32 + lr) * D;
-        } else {
-            int64_t i = q0 + lr;
-            i = i < a.lq ? i : a.lq - 1;
-            qp = a.q + bi * a.qnb3 + hi * a.qnb2 + i * a.qnb1;
-        }
-        take_query(qp);
-        if constexpr (LOCAL) __syncthreads();  // every wave's queries read before the ring is filled
-    }
-    // LOCAL (the tiles fit the ring with a buffer to spare): the workgroup
-    // splits the keys and values itself, tile t into buffer t, where the other
-    // form copies the tiles made by attention_tiles_kernel; each tile's values
-    // go first as they stand into the spare buffer, rows read as float4, and
-    // are transposed from there.
-    if constexpr (LOCAL && !kBatch) {
-        const float *vg = static_cast<const float *>(a.v) + bi * a.vnb3 + kh * a.vnb2;
-        float *vt = reinterpret_cast<float *>(sbuf + (NS - 1) * kStride);  // [KB][D + 4]
-        for (int64_t t = 0; t < nk; ++t) {
-            _Float16 *rec = reinterpret_cast<_Float16 *>(sbuf + t * kStride);
-            split_keys<D, KB>(a, bi, kh, t, rec);
-            for (int idx = tid; idx < KB * (D / 4); idx += 256) {
-                const int j = idx / (D / 4), c4 = idx - j * (D / 4);
-                const int64_t key = t * KB + j;
-                float4v x = float4v{};
-                if (key < a.lk) x = *reinterpret_cast<const float4v *>(vg + key * a.vnb1 + 4 * c4);
-                *reinterpret_cast<float4v *>(vt + j * (D + 4) + 4 * c4) = x;
-            }
-            __syncthreads();
-            split_values<D, KB>([&](int j, int dim) { return vt[j * (D + 4) + dim]; }, rec);
-            __syncthreads();
-        }
+    {
+        const int64_t i = q0 + lr < a.lq ? q0 + lr : a.lq - 1;
+        const float *qp = a.q + bi * a.qnb3 + hi * a.qnb2 + i * a.qnb1;
+        split_query<D, KB>([&](int, int, int dim) { return qp[dim]; }, a.scale, g, qh, ql);
     }
     float16v oh[S::kDvt], ol[S::kDvt];
 #pragma unroll
@@ -1391,7 +1333,6 @@ __global__ __launch_bounds__(256, OCC) void attention_split_kernel(AttentionArgs
     // NS - 1 is.
     constexpr int kAhead = PIPE ? NS - 2 : NS - 1;
     const auto sync = [&](int64_t t) {
-        if constexpr (LOCAL) return;  // every tile in LDS since the start
         // The wave's copies of tile t are done once at most kAhead - 1
         // tiles' copies are outstanding after them (none, near the end);
         // every wave's are, past the barrier, which also ends every wave's
@@ -1410,7 +1351,7 @@ __global__ __launch_bounds__(256, OCC) void attention_split_kernel(AttentionArgs
     half8 kah[S::kSteps][S::kTiles], kal[S::kSteps][S::kTiles];
     half8 vah[S::kTiles][2][S::kDvt], val[S::kTiles][2][S::kDvt];
     const auto read_keys = [&](int64_t t) {
-        const _Float16 *kbuf = reinterpret_cast<const _Float16 *>(sbuf + (t % NS) * kStride);
+        const _Float16 *kbuf = reinterpret_cast<const _Float16 *>(sbuf + (t % NS) * S::kRecord);
 #pragma unroll
         for (int st = 0; st < S::kSteps; ++st)
 #pragma unroll
@@ -1422,7 +1363,7 @@ __global__ __launch_bounds__(256, OCC) void attention_split_kernel(AttentionArgs
             }
     };
     const auto read_values = [&](int64_t t) {
-        const _Float16 *vbuf = reinterpret_cast<const _Float16 *>(sbuf + (t % NS) * kStride) + S::kValues;
+        const _Float16 *vbuf = reinterpret_cast<const _Float16 *>(sbuf + (t % NS) * S::kRecord) + S::kValues;
 #pragma unroll
         for (int u = 0; u < S::kTiles; ++u)
 #pragma unroll
@@ -1434,65 +1375,19 @@ __global__ __launch_bounds__(256, OCC) void attention_split_kernel(AttentionArgs
                     if (!S::kPackV || dt < S::kDvt - 1) val[u][c][dt] = *reinterpret_cast<const half8 *>(vp + S::kPlaneV);
                 }
     };
-    // S^T of the tile whose keys read_keys read.
     const auto scores = [&](float16v (&sh)[S::kTiles], float16v (&sx)[S::kTiles]) {
-#pragma unroll
-        for (int u = 0; u < S::kTiles; ++u) {
-            sh[u] = float16v{};
-            sx[u] = float16v{};
-        }
-#pragma unroll
-        for (int st = 0; st < S::kSteps; ++st)
-#pragma unroll
-            for (int u = 0; u < S::kTiles; ++u) {
-                sh[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kah[st][u], qh[st], sh[u], 0, 0, 0);
-                sx[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kah[st][u], ql[st], sx[u], 0, 0, 0);
-                if (!S::kHalfStep || st < S::kSteps - 1)
-                    sx[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kal[st][u], qh[st], sx[u], 0, 0, 0);
-            }
+        score_products<D, KB>(kah, kal, qh, ql, sh, sx);
     };
-    // O^T += V^T P^T of tile t, a chunk of 16 keys at a time: the lane's
-    // eight exponentials 8 c .. 8 c + 7 of a tile of 32 are its operand B.
     const auto values = [&](const float (&p)[S::kTiles][16]) {
-#pragma unroll
-        for (int u = 0; u < S::kTiles; ++u)
-#pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                // The exponentials (2^11 times, below 2^15) as two FP16 parts,
-                // the second the remainder of the first, in pairs.
-                half8 ph, pl;
-#pragma unroll
-                for (int j = 0; j < 8; j += 2) {
-                    const float x0 = p[u][8 * c + j], x1 = p[u][8 * c + j + 1];
-                    const auto h = __builtin_amdgcn_cvt_pkrtz(x0, x1);
-                    // x - h, each one v_fma_mix_f32 (its -1 unknown to the
-                    // compiler, which would make it a conversion and a
-                    // subtraction).
-                    const auto r = __builtin_amdgcn_cvt_pkrtz(__builtin_fmaf(static_cast<float>(h[0]), minus_one, x0),
-                                                              __builtin_fmaf(static_cast<float>(h[1]), minus_one, x1));
-                    ph[j] = h[0];
-                    ph[j + 1] = h[1];
-                    pl[j] = r[0];
-                    pl[j + 1] = r[1];
-                }
-#pragma unroll
-                for (int dt = 0; dt < S::kDvt; ++dt) {
-                    oh[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vah[u][c][dt], ph, oh[dt], 0, 0, 0);
-                    oh[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vah[u][c][dt], pl, oh[dt], 0, 0, 0);
-                    if (!S::kPackV || dt < S::kDvt - 1)  // the packed tile's low parts are rows of vah
-                        ol[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(val[u][c][dt], ph, ol[dt], 0, 0, 0);
-                }
-            }
+        value_products<D, KB>(p, vah, val, oh, ol, minus_one);
     };
 
     // The first kAhead tiles on their way, once the queries are in; then
     // every tile but the last (with PIPE, the next one's scores beside it),
     // and the last, masked where it is not full.
-    if constexpr (!LOCAL) {
 #pragma unroll
-        for (int st = 0; st < kAhead; ++st) {
-            if (st < nk) issue(st, st);
-        }
+    for (int st = 0; st < kAhead; ++st) {
+        if (st < nk) issue(st, st);
     }
     const auto last = [&](float16v (&sh)[S::kTiles], float16v (&sx)[S::kTiles]) {
         float p[S::kTiles][16];
@@ -1559,17 +1454,7 @@ __global__ __launch_bounds__(256, OCC) void attention_split_kernel(AttentionArgs
         last(sh, sx);
     }
 
-    // The query's sum over its two lanes, or from the rows of ones (the same
-    // on both); lane holds O^T[32 dt + 8 (e / 4) + 4 g + e % 4][lr], and the
-    // values' 2^-4 comes back with the reciprocal.  The packed tile's low
-    // parts are kVLast rows, kVLast / 2 elements, below its high parts.
-    double sum;
-    if constexpr (S::kSumRow) {
-        sum = static_cast<double>(oh[S::kDvt - 1][S::kVLast]) * 16.0;
-    } else {
-        sum = l;
-        sum += __shfl_xor(sum, 32, 64);
-    }
+    const double sum = sum_of<D, KB>(l, oh);
     const auto low = [&](int dt, int e) {
         return S::kPackV && dt == S::kDvt - 1 ? oh[dt][e + S::kVLast / 2] : ol[dt][e];
     };
@@ -1598,22 +1483,211 @@ __global__ __launch_bounds__(256, OCC) void attention_split_kernel(AttentionArgs
             }
         return;
     }
-    const float reciprocal = static_cast<float>(1.0 / sum);
-    float *out = a.y + bi * a.ynb3 + i * a.ynb2 + hi * a.ynb1;
+    store_query<D, KB>(sum, oh, ol, g, a.y + bi * a.ynb3 + i * a.ynb2 + hi * a.ynb1);
+}
+
+// Few keys (cross-attention's 77 or 154), whose tiles all fit a CU's LDS: one
+// launch, a workgroup's waves splitting the head's keys and values into LDS
+// once and each then taking 32 queries after 32 on its own, the next ones'
+// rows on their way while it computes -- no barrier after the first, and no
+// wait for memory but the first.  Heads of up to 96 dimensions take eight
+// waves, larger ones four, whose accumulators need the registers.
+//
+// What bounds it: HBM and the first wait (4 .. 5 us of load, split and
+// barrier).  A workgroup of its own for every 128 queries, which splits the
+// keys and values each time, took 25.9 us for 6240 queries of 16 heads of 40
+// and 77 keys (32 MB, 6.3 us at a copy's rate); this form 16.1, of which a wave's
+// second 32 queries are about 5 (a chain of products, maximum, exponentials and
+// products with one other wave on the SIMD beside it).  Tiles of 64 and 96 keys,
+// for longer chains side by side: 20.3 and 23.3 us (registers spilled).
+template <int D>
+struct Few {
+    static constexpr int kKeys = D <= 64 ? 32 : 32;  // a tile's
+    static constexpr int kWaves = D <= 96 ? 8 : 4;    // the most waves of a workgroup
+    static constexpr bool kAhead = D <= 80;  // the next queries' rows loaded ahead, where the registers allow it
+    static constexpr int kRecord = Split<D, kKeys>::kRecord;
+    static constexpr int kMostTiles = 160 * 1024 / kRecord < 192 / kKeys ? 160 * 1024 / kRecord : 192 / kKeys;
+};
+
+template <int D>
+__global__ __launch_bounds__(64 * Few<D>::kWaves, Few<D>::kWaves / 4) void attention_few_kernel(AttentionArgs a,
+                                                                                          uint32_t per_head) {
+    constexpr int KB = Few<D>::kKeys;
+    using S = Split<D, KB>;
+    const int kThreads = static_cast<int>(blockDim.x);
+    const int waves = kThreads / 64;
+    extern __shared__ __attribute__((aligned(1024))) char sbuf[];  // nk records
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 31;
+    const int g = lane >> 5;
+    float minus_one;
+    asm("s_mov_b32 %0, -1.0" : "=s"(minus_one));
+
+    // The heads of a block of queries, whose rows of queries and of the output
+    // lie side by side in memory and share lines, on consecutive blocks of one
+    // XCD.
+    const uint32_t b = xcd_swizzle(blockIdx.x, gridDim.x);
+    const uint32_t heads = static_cast<uint32_t>(a.b * a.h);
+    const uint32_t slot = b / heads;
+    const uint32_t bh = b - slot * heads;
+    const int64_t hi = bh % a.h;
+    const int64_t bi = bh / a.h;
+    const int64_t kh = hi / (a.h / a.hk);
+    const int nk = static_cast<int>((a.lk + KB - 1) / KB);
+    const int64_t wave_tiles = (a.lq + 31) / 32;
+    const int64_t step = static_cast<int64_t>(per_head) * waves;
+    int64_t wt = static_cast<int64_t>(slot) * waves + wave;
+
+    // A wave tile's queries as split_query reads them: the lane's eight
+    // dimensions of each step (the last step's eight again where its upper
+    // half holds those below).
+    const float *qg = a.q + bi * a.qnb3 + hi * a.qnb2;
+    float4v qv[S::kSteps][2];
+    const auto load_queries = [&](int64_t t) {
+        const int64_t i = 32 * t + lr < a.lq ? 32 * t + lr : a.lq - 1;
+        const float *p = qg + i * a.qnb1;
 #pragma unroll
-    for (int dt = 0; dt < S::kDvt; ++dt)
+        for (int st = 0; st < S::kSteps; ++st) {
+            const int dim = 16 * st + 8 * (S::kHalfStep && st == S::kSteps - 1 ? 0 : g);
+            qv[st][0] = *reinterpret_cast<const float4v *>(p + dim);
+            qv[st][1] = *reinterpret_cast<const float4v *>(p + dim + 4);
+        }
+    };
+    if (Few<D>::kAhead && wt < wave_tiles) load_queries(wt);
+
+    // The keys, a thread a float4 of a key, and the values, a thread four keys
+    // by four dimensions, transposed in its registers.
+    {
+        const float *kg = static_cast<const float *>(a.k) + bi * a.knb3 + kh * a.knb2;
+        const float *vg = static_cast<const float *>(a.v) + bi * a.vnb3 + kh * a.vnb2;
+        const auto load = [&](const float *p, int64_t row, int key, int c4) {
+            float4v x = float4v{};
+            if (key < a.lk) x = *reinterpret_cast<const float4v *>(p + key * row + 4 * c4);
+            return x;
+        };
+        const auto split4 = [](float4v x, half4a &h, half4a &l) {
 #pragma unroll
-        for (int e4 = 0; e4 < 4; ++e4) {
-            const int dim = 32 * dt + 8 * e4 + 4 * g;
-            if (dim < D) {
-                float4v r;
+            for (int r = 0; r < 4; ++r) {
+                _Float16 hh, ll;
+                split_part(x[r] * kSplitDown, hh, ll);
+                h[r] = hh;
+                l[r] = ll;
+            }
+        };
+        const auto put_key = [&](int key, int c4, float4v x) {
+            _Float16 *rec = reinterpret_cast<_Float16 *>(sbuf + (key / KB) * S::kRecord);
+            const int j = key % KB;
+            half4a h, l;
+            split4(x, h, l);
+            *reinterpret_cast<half4a *>(rec + j * S::kLdk + 4 * c4) = h;
+            if (4 * c4 < S::kLdkl) *reinterpret_cast<half4a *>(rec + S::kPlaneK + j * S::kLdkl + 4 * c4) = l;
+            if (S::kHalfStep && 4 * c4 >= D - 8) *reinterpret_cast<half4a *>(rec + j * S::kLdk + 4 * c4 + 8) = l;
+        };
+        // Keys 4 kq .. + 3 are columns c .. c + 3 of their tile (key_of_column).
+        const auto put_values = [&](int kq, int c4, const float4v (&x)[4]) {
+            _Float16 *vh = reinterpret_cast<_Float16 *>(sbuf + (kq / (KB / 4)) * S::kRecord) + S::kValues;
+            const int j = 4 * (kq % (KB / 4));
+            const int c = (j & ~15) + 8 * ((j >> 2) & 1) + 4 * ((j >> 3) & 1);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    r[u] = ((oh[dt][4 * e4 + u] + low(dt, 4 * e4 + u) * kPartDown) * 16.0f) * reciprocal;
-                }
-                *reinterpret_cast<float4v *>(out + dim) = r;
+            for (int r = 0; r < 4; ++r) {
+                const int dim = 4 * c4 + r;
+                half4a h, l;
+                split4(float4v{x[0][r], x[1][r], x[2][r], x[3][r]}, h, l);
+                *reinterpret_cast<half4a *>(vh + dim * S::kLdv + c) = h;
+                if (dim < S::kDvlo) *reinterpret_cast<half4a *>(vh + S::kPlaneV + dim * S::kLdv + c) = l;
+                if (S::kPackV && dim >= D - S::kVLast)
+                    *reinterpret_cast<half4a *>(vh + (dim + S::kVLast) * S::kLdv + c) = l;
+            }
+        };
+        const int keys = nk * KB;
+        constexpr int kBatch = 4;
+        for (int base = tid; base < keys * (D / 4); base += kThreads * kBatch) {
+            float4v x[kBatch];
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                const int idx = base + kThreads * u;
+                const int key = idx / (D / 4);
+                x[u] = load(kg, a.knb1, key, idx - key * (D / 4));
+            }
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                const int idx = base + kThreads * u;
+                const int key = idx / (D / 4);
+                if (idx < keys * (D / 4)) put_key(key, idx - key * (D / 4), x[u]);
             }
         }
+        for (int idx = tid; idx < keys / 4 * (D / 4); idx += kThreads) {
+            const int kq = idx / (D / 4);
+            const int c4 = idx - kq * (D / 4);
+            float4v x[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x[u] = load(vg, a.vnb1, 4 * kq + u, c4);
+            put_values(kq, c4, x);
+        }
+        if constexpr (S::kSumRow) {
+            // The rows of 2^-4 that sum the exponentials.
+            for (int idx = tid; idx < nk * 8 * (KB / 4); idx += kThreads) {
+                const int row = D + S::kVLast + idx / (KB / 4) % 8;
+                _Float16 *vh = reinterpret_cast<_Float16 *>(sbuf + idx / (8 * (KB / 4)) * S::kRecord) + S::kValues;
+                const _Float16 one = static_cast<_Float16>(kSplitDown);
+                *reinterpret_cast<half4a *>(vh + row * S::kLdv + 4 * (idx % (KB / 4))) = half4a{one, one, one, one};
+            }
+        }
+    }
+    __syncthreads();
+
+    for (; wt < wave_tiles; wt += step) {
+        if (!Few<D>::kAhead) load_queries(wt);
+        half8 qh[S::kSteps], ql[S::kSteps];
+        split_query<D, KB>([&](int st, int j, int) { return qv[st][j >> 2][j & 3]; }, a.scale, g, qh, ql);
+        if (Few<D>::kAhead && wt + step < wave_tiles) load_queries(wt + step);
+        float16v oh[S::kDvt], ol[S::kDvt];
+#pragma unroll
+        for (int c = 0; c < S::kDvt; ++c) {
+            oh[c] = float16v{};
+            ol[c] = float16v{};
+        }
+        float m = -INFINITY;
+        double l = 0.0;
+        for (int t = 0; t < nk; ++t) {
+            const _Float16 *kbuf = reinterpret_cast<const _Float16 *>(sbuf + t * S::kRecord);
+            const _Float16 *vbuf = kbuf + S::kValues;
+            half8 kah[S::kSteps][S::kTiles], kal[S::kSteps][S::kTiles];
+#pragma unroll
+            for (int st = 0; st < S::kSteps; ++st)
+#pragma unroll
+                for (int u = 0; u < S::kTiles; ++u) {
+                    const int row = 32 * u + lr, at = 16 * st + 8 * g;
+                    kah[st][u] = *reinterpret_cast<const half8 *>(kbuf + row * S::kLdk + at);
+                    if (!S::kHalfStep || st < S::kSteps - 1)
+                        kal[st][u] = *reinterpret_cast<const half8 *>(kbuf + S::kPlaneK + row * S::kLdkl + at);
+                }
+            float16v sh[S::kTiles], sx[S::kTiles];
+            score_products<D, KB>(kah, kal, qh, ql, sh, sx);
+            float p[S::kTiles][16];
+            const int valid = static_cast<int>(a.lk) - t * KB;
+            const float shift = split_max<true, !S::kSumRow, S::kTiles, S::kDvt>(sh, sx, p, m, l, oh, ol, valid, g);
+            split_exp<!S::kSumRow, S::kTiles>(p, shift, l);
+            half8 vah[S::kTiles][2][S::kDvt], val[S::kTiles][2][S::kDvt];
+#pragma unroll
+            for (int u = 0; u < S::kTiles; ++u)
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+#pragma unroll
+                    for (int dt = 0; dt < S::kDvt; ++dt) {
+                        const _Float16 *vp = vbuf + (32 * dt + lr) * S::kLdv + 32 * u + 16 * c + 8 * g;
+                        vah[u][c][dt] = *reinterpret_cast<const half8 *>(vp);
+                        if (!S::kPackV || dt < S::kDvt - 1)
+                            val[u][c][dt] = *reinterpret_cast<const half8 *>(vp + S::kPlaneV);
+                    }
+            value_products<D, KB>(p, vah, val, oh, ol, minus_one);
+        }
+        const double sum = sum_of<D, KB>(l, oh);
+        const int64_t i = 32 * wt + lr;
+        if (i < a.lq) store_query<D, KB>(sum, oh, ol, g, a.y + bi * a.ynb3 + i * a.ynb2 + hi * a.ynb1);
+    }
 }
 
 // The key splits of the split form merged, query by query: each split's sum
@@ -1664,6 +1738,14 @@ struct KeySplits {
     int64_t splits, per;
 };
 
+// Whether the keys are few enough for attention_few_kernel: their tiles fit
+// a CU's LDS, six of them at most (192 keys; beyond, the tiles' own launch is
+// repaid by the workgroups that share it).
+template <int D>
+bool few_keys(const AttentionArgs &a) {
+    return ceil_div(a.lk, Few<D>::kKeys) <= Few<D>::kMostTiles;
+}
+
 template <int D>
 KeySplits key_splits(const AttentionArgs &a) {
     using SH = SplitShape<D>;
@@ -1671,7 +1753,7 @@ KeySplits key_splits(const AttentionArgs &a) {
     const int64_t nk = ceil_div(a.lk, SH::kKeys);
     const int64_t blocks = ceil_div(a.lq, S::kQueries) * a.h * a.b;
     int64_t sp = 1;
-    if (nk >= SH::kStages && blocks > 0 && blocks < compute_units()) {  // the tiles' launch (not LOCAL)
+    if (!few_keys<D>(a) && blocks > 0 && blocks < compute_units()) {
         sp = compute_units() / blocks;
         sp = sp < nk / 2 ? sp : nk / 2;
         sp = sp < 1 ? 1 : sp;
@@ -1712,45 +1794,40 @@ size_t split_work(const AttentionArgs &a) {
     return ks.splits > 1 ? tiles + key_partial_layout(a, ks.splits).bytes : tiles;
 }
 
-template <int D, bool LOCAL>
-hipError_t launch_split_t(AttentionArgs a, void *work, hipStream_t stream) {
-    using SH = SplitShape<D>;
-    using S = Split<D, SH::kKeys>;
-    a.qblocks = ceil_div(a.lq, S::kQueries);
-    const size_t lds = static_cast<size_t>(SH::kStages) * (LOCAL ? S::kLocalBuffer : S::kRecord);
-    static const hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void *>(&attention_split_kernel<D, SH::kKeys, SH::kStages, SH::kOcc, SH::kPipe, LOCAL>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+// Few keys: a workgroup a CU, or two where LDS holds both and there are wave
+// tiles for them; the wave tiles of a head shared out evenly.
+template <int D>
+hipError_t launch_few(const AttentionArgs &a, hipStream_t stream) {
+    using F = Few<D>;
+    const int64_t heads = a.h * a.b;
+    const size_t lds = static_cast<size_t>(ceil_div(a.lk, F::kKeys)) * F::kRecord;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&attention_few_kernel<D>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       F::kMostTiles * F::kRecord);
     if (attr != hipSuccess) return attr;
-    const int64_t nk = ceil_div(a.lk, SH::kKeys);
-    const KeySplits ks = LOCAL ? KeySplits{1, nk} : key_splits<D>(a);
-    KeyPartial part{};
-    if (ks.splits > 1) {
-        char *base = static_cast<char *>(work) + split_tiles_bytes<D>(a);
-        const KeyPartialLayout k = key_partial_layout(a, ks.splits);
-        part.l = reinterpret_cast<double *>(base + k.l);
-        part.m = reinterpret_cast<float *>(base + k.m);
-        part.o = reinterpret_cast<float *>(base + k.o);
-    }
-    dim3 grid(static_cast<uint32_t>(a.qblocks * a.h * a.b * ks.splits)), block(256);
+    // Eight waves a CU share the heads' wave tiles in as few rounds as they can,
+    // each about as many.  Workgroups of eight waves, or of four where those
+    // would leave half the CUs without one (1024 queries of 16 heads of 80, 64
+    // workgroups of eight: 12.9 us, of four 11.9; 988 of 40 heads of 64, 160 of
+    // eight: 13.0, of four 19.1).
+    const int64_t wave_tiles = ceil_div(a.lq, 32);
+    const int64_t waves = F::kWaves == 8 && 2 * heads * ceil_div(wave_tiles, 8) >= compute_units() ? 8 : 4;
+    const int64_t most = 8 * compute_units() / heads > waves ? 8 * compute_units() / heads : waves;
+    const int64_t rounds = ceil_div(wave_tiles, most);
+    const int64_t per_head = ceil_div(ceil_div(wave_tiles, rounds), waves);
+    if (heads * per_head >= (int64_t{1} << 22)) return hipErrorInvalidValue;
     KernelScope scope("attention", stream);
-    SDHIP_LAUNCH((attention_split_kernel<D, SH::kKeys, SH::kStages, SH::kOcc, SH::kPipe, LOCAL>), grid, block, lds,
-                 stream, a, static_cast<const char *>(work), ks.splits, ks.per, part);
-    if (ks.splits > 1) {
-        SDHIP_LAUNCH(split_combine_kernel, dim3(static_cast<uint32_t>(ceil_div(a.b * a.h * a.lq, 4))), block, 0,
-                     stream, a, ks.splits, part);
-    }
+    SDHIP_LAUNCH(attention_few_kernel<D>, dim3(static_cast<uint32_t>(heads * per_head)), dim3(static_cast<uint32_t>(64 * waves)), lds,
+                 stream, a, static_cast<uint32_t>(per_head));
     return hipGetLastError();
 }
 
 template <int D>
 hipError_t launch_split(AttentionArgs a, void *work, hipStream_t stream) {
     using SH = SplitShape<D>;
+    using S = Split<D, SH::kKeys>;
+    if (few_keys<D>(a)) return launch_few<D>(a, stream);
     const int64_t nk = ceil_div(a.lk, SH::kKeys);
-    // Keys and values that fit the ring with a buffer to spare
-    // (cross-attention's 77 at heads of up to 64): each workgroup splits them
-    // itself, with no launch before it.
-    if (nk < SH::kStages) return launch_split_t<D, true>(a, nullptr, stream);
     // The tiles' grid is one dimension of 256-thread blocks: under 2^24 of
     // them (a work buffer of 14 KB or more a tile, past 230 GB, before that).
     if (nk * a.b * a.hk >= (int64_t{1} << 24)) return hipErrorInvalidValue;
@@ -1761,7 +1838,30 @@ hipError_t launch_split(AttentionArgs a, void *work, hipStream_t stream) {
         const hipError_t err = hipGetLastError();
         if (err != hipSuccess) return err;
     }
-    return launch_split_t<D, false>(a, work, stream);
+    a.qblocks = ceil_div(a.lq, S::kQueries);
+    const size_t lds = static_cast<size_t>(SH::kStages) * S::kRecord;
+    static const hipError_t attr = hipFuncSetAttribute(
+        reinterpret_cast<const void *>(&attention_split_kernel<D, SH::kKeys, SH::kStages, SH::kOcc, SH::kPipe>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+    if (attr != hipSuccess) return attr;
+    const KeySplits ks = key_splits<D>(a);
+    KeyPartial part{};
+    if (ks.splits > 1) {
+        char *base = static_cast<char *>(work) + split_tiles_bytes<D>(a);
+        const KeyPartialLayout k = key_partial_layout(a, ks.splits);
+        part.l = reinterpret_cast<double *>(base + k.l);
+        part.m = reinterpret_cast<float *>(base + k.m);
+        part.o = reinterpret_cast<float *>(base + k.o);
+    }
+    dim3 grid(static_cast<uint32_t>(a.qblocks * a.h * a.b * ks.splits)), block(256);
+    KernelScope scope("attention", stream);
+    SDHIP_LAUNCH((attention_split_kernel<D, SH::kKeys, SH::kStages, SH::kOcc, SH::kPipe>), grid, block, lds,
+                 stream, a, static_cast<const char *>(work), ks.splits, ks.per, part);
+    if (ks.splits > 1) {
+        SDHIP_LAUNCH(split_combine_kernel, dim3(static_cast<uint32_t>(ceil_div(a.b * a.h * a.lq, 4))), block, 0,
+                     stream, a, ks.splits, part);
+    }
+    return hipGetLastError();
 }
 
 template <int D, int QT, int KB>

@@ -312,3 +312,28 @@ def test_attention512(gpu, c, spread):
     print(f"attention {c} spread {spread}: {errors}")
     assert errors[""] <= BOUND
     assert errors[""] <= 1.5 * errors["attention_fp32=1"] + 1e-7
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,lq,lk,h,hk,b", [
+    (40, 2081, 77, 8, 8, 2),    # workgroups of eight waves, ragged queries
+    (40, 33, 97, 3, 1, 1),      # two wave tiles, one key past a tile, heads sharing keys
+    (32, 5000, 1, 16, 16, 2),   # several rounds of queries, one key
+    (64, 300, 192, 2, 2, 1),    # the most keys
+    (80, 1000, 160, 2, 2, 1),   # the most tiles that fit LDS, workgroups of four
+    (80, 64, 161, 2, 2, 1),     # one key more: the tiles' launch
+    (96, 700, 129, 4, 2, 1),
+    (128, 31, 96, 2, 2, 1),
+    (160, 100, 96, 2, 2, 1),
+    (160, 65, 97, 2, 2, 1),     # past LDS
+], ids=str)
+def test_attention_few_keys(gpu, d, lq, lk, h, hk, b):
+    """Keys whose tiles fit a CU's LDS: every workgroup splits them once and
+    its waves take query after query -- at the edges of the tiles, of the
+    rounds and of the rule, within the bound of float64."""
+    q, k, v, y, scale = attention_case(gpu, d, lq, lk, h, hk, b, False, seed=d + lq + lk, dist="normal")
+    exact, mag = orc.exact_attention(q, k, v, scale)
+    err = orc.metric(y, exact, mag)
+    print(f"few keys {(d, lq, lk, h, hk, b)}: {err:.3g}")
+    assert np.isfinite(y).all()
+    assert err <= BOUND
