@@ -766,15 +766,12 @@ def unet_step_line(dev, args):
 # those of the configurations' work units, restated:
 #   cfg1  Y = X W^T + b, X 2x4096x320 f32, W 320x320 f16: X 10.49 MB + W 0.20 +
 #         b + Y 10.49 = 21.18 MB (AI 79: HBM-bound at the split-FP16 rate)
-#   cfg2  the 36 products of 320x320 by 512 tiles: 2 x 36 x 320 x 320 x 512
-#         = 3.775 GFLOP a call on the FP16 MFMA, three MFMAs a product, against
-#         the raw 2.5 PF (and the split's 833 TF effective); the op's
-#         direct-equivalent 15.10 GFLOP against the target of 1.5 x 2.5 PF.
-#         Beside it, the products' bytes (U and V read once as two FP16
-#         planes, 36 x 2 x 2 x (320 + 512) x 320 = 38.34 MB; M written once,
-#         36 x 4 x 320 x 512 = 23.59 MB) against 8 TB/s, and the whole op's
-#         counter bytes against its own algorithmic 33.3 MB (input 10.49 MB,
-#         FP16 weights 1.84, bias, residual 10.49, output 10.49)
+#   cfg2  the 3x3 convolution, whose products the library takes directly at
+#         this size: 15.10 GFLOP a call on the FP16 MFMA, two MFMAs a product,
+#         against the raw 2.5 PF (and the split's 1250 TF effective) and the
+#         target of 1.5 x 2.5 PF.  Beside it, the bytes of the op (input 10.49
+#         MB, FP16 weights 1.84, bias, residual 10.49, output 10.49) against
+#         8 TB/s, and its counter bytes against them
 #   cfg3a F(2x2) of 8x8 maps: the products kernel reads the FP16 weights,
 #         1280x1280x9x2 = 29.49 MB (it makes U in registers)
 #   cfg3b 1x1 conv 2x640x1024 -> 1280: 3.355 GFLOP
@@ -784,9 +781,9 @@ def unet_step_line(dev, args):
 CONFIGS = {
     "cfg1_linear": dict(workload="cfg1", unit="TFLOP/s", kernels=("mul_mat",), bound="hbm", amount=21.18e6,
                         peak=PEAK_HBM),
-    "cfg2_winograd4": dict(workload="cfg2", unit="TFLOP/s", kernels=("winograd4.products",), bound="mfma",
-                           amount=2.0 * 36 * 320 * 320 * 512, peak=PEAK_FP16_MFMA, split=3,
-                           hbm_bytes=36 * 2 * 2 * (320 + 512) * 320 + 36 * 4 * 320 * 512.0,
+    "cfg2_winograd4": dict(workload="cfg2", unit="TFLOP/s", kernels=("conv3x3.products",), bound="mfma",
+                           amount=2.0 * 9 * 320 * 320 * 2 * 64 * 64, peak=PEAK_FP16_MFMA, split=2,
+                           hbm_bytes=(3 * 2 * 320 * 64 * 64 + 320) * 4 + 320 * 320 * 9 * 2.0,
                            op_bytes=(3 * 2 * 320 * 64 * 64 + 320) * 4 + 320 * 320 * 9 * 2.0, op_target=1.5),
     "cfg3a_winograd2_gn_silu": dict(workload="cfg3a", unit="TFLOP/s", kernels=("winograd2.products",), bound="hbm",
                                     amount=1280 * 1280 * 9 * 2.0, peak=PEAK_HBM),
@@ -901,14 +898,14 @@ def main():
                           "tflops": round(flops / ms / 1e9, 3) if flops else None}), flush=True)
         return
 
-    # The headline: configs[1], F(4x4) with bias and residual fused.
+    # The headline: configs[1], the reference's F(4x4), with bias and residual fused.
     _, _, path = conv_workload(dev, 2, 320, 64, 64, 320, 3, 1, seed=2)
     assert path == 4, f"configs[1] takes path {path}, not F(4x4)"
     head, ms, work, kt = measure_config(dev, "cfg2_winograd4", args)
     value = work / ms / 1e9
     fp32 = sdhip.get_tuning("winograd_fp32") == 1
     roof = dict(head["roofline"])
-    roof["mfma"] = "v_mfma_f32_16x16x4_f32" if fp32 else "v_mfma_f32_32x32x16_f16, 3 per product (split FP16)"
+    roof["mfma"] = "v_mfma_f32_16x16x4_f32" if fp32 else "v_mfma_f32_16x16x32_f16, 2 per product (split FP16)"
     roof["kernels_us"] = {k: round(v[0] * 1e3, 2) for k, v in kt.items()}
     roof["direct_eq_vs_fp16_peak"] = round(value / PEAK_FP16_MFMA, 4)
     configs = {"cfg2_winograd4": head}
@@ -949,8 +946,9 @@ def main():
         "vs_baseline": None,
         "dtype": "f32",
         "data": "synthetic",
-        "config": {"workload": "configs[1]: SD1.5 ResNet 3x3 conv [2,320,64,64]->320, pad 1, Winograd F(4x4,3x3), "
-                               "FP16 weights ~N(0,0.02), fused bias + residual add",
+        "config": {"workload": "configs[1]: SD1.5 ResNet 3x3 conv [2,320,64,64]->320, pad 1 (Winograd F(4x4,3x3) "
+                               "in the reference, direct products here), FP16 weights ~N(0,0.02), fused bias + "
+                               "residual add",
                    "parallelism": "none (1 GPU)"},
         "roofline": roof,
         "configs": configs,

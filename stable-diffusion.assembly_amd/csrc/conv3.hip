@@ -1,0 +1,658 @@
+// 3x3 convolutions at stride 1 of FP16 kernels, directly: an implicit product
+// of the nine taps on v_mfma_f32_16x16x32_f16, one pass over the image, for the
+// sizes where F(4x4, 3x3) spends its time on the launches and the bytes between
+// its transforms and products rather than on the products it saves.
+//
+// Precision.  The weights are exact FP16 operands.  Each input x is scaled by
+// an exact power of two 2^-E and taken as h = fp16(x), l = fp16(x - h), two
+// MFMAs a product: 22 bits of x.  E is the workgroup's own and follows its
+// inputs as they come: it brings the greatest |x| so far into [2^13, 2^15), and
+// where a later chunk of channels passes that, the sums are rescaled (exactly)
+// and E raised.  So l is normal for every x within 2^17 of the greatest and
+// 2^-40 of that greatest off at most below, at any magnitude, and no pass over
+// the image is needed before the products.  Against 64 bits this is nearer than
+// F(4x4), whose transforms round and amplify.
+//
+// Shape.  A workgroup takes tiles of kRows x 16 outputs of an image by kOc
+// output channels.  Its first waves compute, WP x WO x KS of them: WP groups of
+// RW rows, WO groups of 16 NO channels, KS groups of input channels (each its
+// own chunk of 32 at a time, their sums added through LDS at the end), so that
+// small images fill the CUs with tiles whose waves still hold 64 or more
+// accumulators.  Its last four waves fetch: a chunk's inputs, with their
+// border, two chunks ahead into registers, their greatest magnitude found, and
+// a chunk ahead split into LDS, [part][position][32 channels], two buffers, one
+// barrier a chunk.  So a computing wave waits for no input: the memory counter
+// is in order, and weights loaded behind inputs from HBM waited for those (kw0
+// of the first version's chunks: 8600 cycles of the 3000 its MFMAs take).
+// A fragment is 16 positions of a row by 32 channels; an input row's serves the
+// three taps above each other of its column.  The weights, laid out as
+// [chunk][tap][oc][32] by a first launch, go from L2 straight into registers, a
+// column of taps ahead.
+//
+// What bounds it (timestamps of the waves, cycles).  A chunk of the 256 x 128
+// form is 9216 cycles of MFMA on each SIMD and takes 11400, the MFMA's rate at
+// 81%; a tile's end, 25000, is HBM's, every CU reading its residual and writing
+// its outputs at once: 128->128 at 520x768 with a residual 595 -> 278 us, of
+// which the bytes (614 MB, once each) are 119 at a copy's rate.  The 64 x 160
+// form has one computing wave on a SIMD, 8300 cycles a pair of chunks of 5760 of
+// MFMA, a start of 10000 and an end of 13500: 320->320 at 64x64, two images,
+// 47.0 -> 35.8 us.  Not faster: two workgroups of 128 x 128 a CU (332 us at
+// 520x768), the residual's lines read ahead by the fetching waves (298), stores
+// past the caches (293), raised priority for either kind of wave.
+// 16-byte piece p of a position's 64 bytes lies at p ^ (position / 4 % 4): the 16
+// positions a fragment read takes are consecutive, so fall in 16 groups of
+// banks.
+
+#include "conv3.h"
+#include "host.h"
+#include "kernels.h"
+#include "profile.h"
+
+namespace sdhip {
+
+namespace {
+
+constexpr int kCols = 16;          // outputs of a tile's row
+constexpr int kPitch = kCols + 2;  // its inputs
+constexpr int kChunk = 32;         // input channels of a chunk
+constexpr int kMostFetch = 4;
+
+template <int RW_, int NO_, int WP_, int WO_, int KS_, int FETCH>
+struct Shape {
+    static constexpr int RW = RW_, NO = NO_, WP = WP_, WO = WO_, KS = KS_;
+    static constexpr int kFetch = FETCH;         // the waves that fetch inputs
+    static constexpr int kWaves = WP * WO * KS;  // that compute
+    static constexpr int kThreads = 64 * (kWaves + kFetch);
+    static constexpr int kRows = RW * WP;
+    static constexpr int kOc = 16 * NO * WO;
+    static constexpr int kPos = (kRows + 2) * kPitch;
+    static constexpr int kItems = kPos * 4 * KS;  // (position, 8 channels)
+    static constexpr int kPer = (kItems + 64 * kFetch - 1) / (64 * kFetch);
+    static constexpr int kPlane = kPos * 2 * kChunk;  // bytes of one part of a chunk
+    static constexpr int kBuffer = KS * 2 * kPlane;
+    static constexpr int kExchange = KS > 1 ? kWaves * RW * NO * 1024 : 0;
+    static constexpr int kLds = 2 * kBuffer > kExchange ? 2 * kBuffer : kExchange;
+    static constexpr int kOwn = RW * NO / KS;  // the tiles of 16 x 16 a wave finishes
+    static_assert(RW * NO % KS == 0 && kFetch <= kMostFetch, "whole tiles a group");
+    static_assert(kLds + 256 <= 160 * 1024, "LDS of a CU");
+};
+
+// 256 outputs by 128 channels, eight computing waves: images of many tiles.
+using Wide = Shape<8, 2, 2, 4, 1, 4>;
+// 64 outputs by 160 channels, four computing waves.
+using Mid = Shape<4, 5, 1, 2, 2, 4>;
+// 64 outputs by 80 channels, four computing waves: few tiles.
+using Narrow = Shape<4, 5, 1, 1, 4, 4>;
+
+struct Conv3Args {
+    WinogradArgs a;
+    const _Float16 *w;  // [chunk][3 kw + kh][oc][32]
+    int32_t chunks, tiles_x, tiles_y;
+    uint32_t tiles;    // of every image and block of output channels
+    uint32_t xbytes;   // an image's, from its first element past its last
+    uint32_t wbytes;
+    int32_t vec_y;     // rows of whole aligned quads: float4 stores
+    uint32_t vec_step;  // bit s: step s's operand in float4
+};
+
+__device__ __forceinline__ int scale_exponent(float m) {
+    int k = 0;
+    frexpf(m, &k);
+    k -= 15;
+    return m > 0.0f ? (k < -110 ? -110 : k) : -110;
+}
+
+// ------------------------------------------------------------------ weights
+
+// [oc][ic][kh][kw] into [ic / 32][3 kw + kh][oc][ic % 32], a thread a kernel.
+__global__ __launch_bounds__(256) void conv3_weights_kernel(const _Float16 *__restrict__ w, int64_t oc, int64_t ic,
+                                                            _Float16 *__restrict__ out) {
+    const int64_t c = static_cast<int64_t>(blockIdx.x) * kChunk + (threadIdx.x & 31);
+    const int64_t o = static_cast<int64_t>(blockIdx.y) * 8 + (threadIdx.x >> 5);
+    if (o >= oc) return;
+    const _Float16 *k = w + (o * ic + c) * 9;
+    _Float16 g[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) g[i] = k[i];
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+        out[((static_cast<int64_t>(blockIdx.x) * 9 + t) * oc + o) * kChunk + (threadIdx.x & 31)] = g[t % 3 * 3 + t / 3];
+}
+
+// ------------------------------------------------------------------ products
+
+// A tile's place.  Consecutive tiles are neighbours of one block of output
+// channels, whose weights and border rows an XCD's L2 then holds.
+struct Place {
+    int img, x0, y0, ob;
+};
+
+template <class S>
+__device__ __forceinline__ Place place_of(const Conv3Args &p, uint32_t tile) {
+    const uint32_t plane_tiles = static_cast<uint32_t>(p.tiles_x * p.tiles_y);
+    const uint32_t spatial = plane_tiles * static_cast<uint32_t>(p.a.n);
+    const uint32_t ob = tile / spatial;
+    uint32_t rest = tile - ob * spatial;
+    const uint32_t img = rest / plane_tiles;
+    rest -= img * plane_tiles;
+    const uint32_t ty = rest / static_cast<uint32_t>(p.tiles_x);
+    return {static_cast<int>(img), static_cast<int>(rest - ty * p.tiles_x) * kCols, static_cast<int>(ty) * S::kRows,
+            static_cast<int>(ob)};
+}
+
+// What the fetching waves hand over beside the buffers.
+struct Handover {
+    float most[2][kMostFetch];  // a chunk's greatest |x|, by wave
+    int e[2];               // a buffer's exponent
+};
+
+// The fetching waves: `count` tiles from `tile` on, `stride` apart.
+template <class S>
+__device__ __forceinline__ void fetch_inputs(const Conv3Args &p, uint32_t tile, uint32_t stride, int count, int steps,
+                                             char *lds, Handover &hand) {
+    constexpr int KS = S::KS;
+    constexpr uint32_t kPast = 0x80000000u;  // past any image (xbytes is below 2^31): reads zero
+    const WinogradArgs &a = p.a;
+    const int tid = static_cast<int>(threadIdx.x) - 64 * S::kWaves;
+    const int lane = tid & 63, wave = tid >> 6;
+    const uint32_t channel = static_cast<uint32_t>(a.xnb2) * 4;  // bytes of a channel's plane
+    // A thread's items: a position of the tile's inputs by 8 channels; their
+    // offsets in the image, past it where the position lies outside.
+    uint32_t from[S::kPer];
+    __amdgpu_buffer_rsrc_t rsrc;
+    const auto locate = [&](uint32_t t) {
+        const Place at = place_of<S>(p, t);
+        rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.x) + static_cast<int64_t>(at.img) * a.xnb3, 0,
+                                                 static_cast<int>(p.xbytes), 0x00020000);
+#pragma unroll
+        for (int u = 0; u < S::kPer; ++u) {
+            const int idx = tid + 64 * S::kFetch * u;
+            const int pos = idx % S::kPos, cg = idx / S::kPos;
+            const int py = pos / kPitch, px = pos - py * kPitch;
+            const int iy = at.y0 + py - a.p1, ix = at.x0 + px - a.p0;
+            const bool in = idx < S::kItems && iy >= 0 && iy < a.ih && ix >= 0 && ix < a.iw;
+            from[u] = in ? static_cast<uint32_t>(iy) * static_cast<uint32_t>(a.xnb1) * 4 + static_cast<uint32_t>(ix) * 4 +
+                               8u * cg * channel
+                         : kPast;
+        }
+    };
+    float x[S::kPer][8];
+    const auto load = [&](int sc) {
+#pragma unroll
+        for (int u = 0; u < S::kPer; ++u) {
+            const int chunk = sc * KS + (tid + 64 * S::kFetch * u) / S::kPos / 4;
+            const uint32_t at = KS > 1 && chunk >= p.chunks ? kPast : from[u];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                x[u][i] = __builtin_bit_cast(
+                    float, __builtin_amdgcn_raw_buffer_load_b32(
+                               rsrc, at, static_cast<uint32_t>(sc * KS * kChunk + i) * channel, 0));
+        }
+    };
+    const auto find_most = [&](int slot) {
+        float m = 0.0f;
+#pragma unroll
+        for (int u = 0; u < S::kPer; ++u)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float v = fabsf(x[u][i]);
+                m = fmaxf(m, v <= 3.402823466e38f ? v : 0.0f);
+            }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+        if (lane == 0) hand.most[slot][wave] = m;
+    };
+    // The chunk's exponent: the tile's so far unless an input passes 2^15
+    // times it, then one bit of room above the chunk's.
+    int erun = -1000;
+    const auto store = [&](int buf, bool first) {
+        float m = hand.most[buf][0];
+#pragma unroll
+        for (int w = 1; w < S::kFetch; ++w) m = fmaxf(m, hand.most[buf][w]);
+        const int e = scale_exponent(m);
+        erun = first || e > erun ? e + 1 : erun;
+        const float f = ldexpf(1.0f, -erun);
+        if (tid == 0) hand.e[buf] = erun;
+#pragma unroll
+        for (int u = 0; u < S::kPer; ++u) {
+            const int idx = tid + 64 * S::kFetch * u;
+            if (idx >= S::kItems) continue;
+            half8 hi, lo;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                _Float16 h, l;
+                split_scaled(x[u][i] * f, h, l);
+                hi[i] = h;
+                lo[i] = l;
+            }
+            const int pos = idx % S::kPos, cg = idx / S::kPos;
+            char *d = lds + buf * S::kBuffer + (cg >> 2) * 2 * S::kPlane + pos * 64 + 16 * ((cg & 3) ^ ((pos >> 2) & 3));
+            *reinterpret_cast<half8 *>(d) = hi;
+            *reinterpret_cast<half8 *>(d + S::kPlane) = lo;
+        }
+    };
+    const int chunks = count * steps;  // of all the tiles
+    int sc = 0;                        // of the chunk in registers
+    const auto advance = [&]() {
+        if (++sc == steps) {
+            sc = 0;
+            tile += stride;
+            locate(tile);
+        }
+        load(sc);
+    };
+    locate(tile);
+    load(0);
+    find_most(0);
+    lds_barrier();
+    store(0, true);
+    if (chunks > 1) advance();
+    lds_barrier();
+    int done = 0;  // chunks of the computing waves' tile
+    for (int g = 0; g < chunks; ++g) {
+        if (g == 0) {  // the second chunk's greatest, beside the first's products
+            if (chunks > 1) find_most(1);
+            lds_barrier();
+        }
+        if (g + 1 < chunks) {
+            store((g + 1) & 1, sc == 0);
+            if (g + 2 < chunks) {
+                advance();
+                find_most(g & 1);
+            }
+        }
+        if (KS > 1 && ++done == steps) {  // the computing waves' exchange
+            done = 0;
+            lds_barrier();
+            lds_barrier();
+        }
+        lds_barrier();
+    }
+}
+
+// A tile's outputs: the groups' sums added, scaled back, the chain, stored.
+template <class S>
+__device__ __forceinline__ void finish(const Conv3Args &p, const Place &at, int oc0, int wp, int wo, int kg, int wave,
+                                       int lane, int erun, float4v (&acc)[S::RW][S::NO], char *lds) {
+    constexpr int RW = S::RW, NO = S::NO, KS = S::KS;
+    const WinogradArgs &a = p.a;
+    const int col = lane & 15, quad = lane >> 4;
+    const int img = at.img, x0 = at.x0, y0 = at.y0;
+    // The groups' sums: each wave writes the tiles it does not finish, and adds
+    // the others' of those it does.
+    float4v v[S::kOwn];
+    if constexpr (KS > 1) {
+        // Over the buffers: every wave's reads of them are done, and a
+        // workgroup of several groups takes one tile.
+        float4v *ex = reinterpret_cast<float4v *>(lds);
+        lds_barrier();
+#pragma unroll
+        for (int j = 0; j < RW * NO; ++j)
+            if (j % KS != kg) ex[(wave * RW * NO + j) * 64 + lane] = acc[j / NO][j % NO];
+        lds_barrier();
+#pragma unroll
+        for (int q = 0; q < S::kOwn; ++q) {
+#pragma unroll
+            for (int g = 0; g < KS; ++g)
+                if (g == kg) v[q] = acc[(KS * q + g) / NO][(KS * q + g) % NO];
+#pragma unroll
+            for (int g = 1; g < KS; ++g) {
+                const int other = (kg + g) % KS * (S::WP * S::WO) + wo * S::WP + wp;
+                v[q] += ex[(other * RW * NO + KS * q + kg) * 64 + lane];
+            }
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < S::kOwn; ++q) v[q] = acc[q / NO][q % NO];
+    }
+
+    // Four or fewer tiles at a time, every load of a step of the chain before any
+    // of its values is used: tile q is outputs x .. x + 3 of a row and channel.
+    constexpr int kGroup = S::kOwn % 4 == 0 ? 4 : 5;
+    static_assert(S::kOwn % kGroup == 0, "whole groups");
+    const float up = ldexpf(1.0f, erun);
+    const int x = x0 + 4 * quad;
+    const int xc = x + 3 < a.ow ? x : static_cast<int>(a.ow) - 4;  // of a quad, where the rows are whole quads
+    const int64_t ynb[4] = {1, a.ynb1, a.ynb2, a.ynb3};
+#pragma unroll
+    for (int q0 = 0; q0 < S::kOwn; q0 += kGroup) {
+        int row[kGroup], och[kGroup];
+        float4v t[kGroup];
+#pragma unroll
+        for (int q = 0; q < kGroup; ++q) {
+            const int j = KS * (q0 + q) + kg;
+            const int yy = y0 + wp * RW + j / NO, oc = oc0 + 16 * (j % NO) + col;
+            row[q] = yy < a.oh ? yy : static_cast<int>(a.oh) - 1;
+            och[q] = oc < a.oc ? oc : static_cast<int>(a.oc) - 1;
+            t[q] = v[q0 + q] * up;
+        }
+        // The values of a tensor at the tiles' outputs: in one piece, or each on
+        // its own.
+        const auto read = [&](const float *from, const int64_t *nb, bool vec, float4v(&o)[kGroup]) {
+            const float *base = from + img * nb[3];
+            if (vec) {
+#pragma unroll
+                for (int q = 0; q < kGroup; ++q)
+                    o[q] = *reinterpret_cast<const float4v *>(base + och[q] * nb[2] + row[q] * nb[1] + xc);
+            } else {
+#pragma unroll
+                for (int q = 0; q < kGroup; ++q)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int xe = x + e < a.ow ? x + e : static_cast<int>(a.ow) - 1;
+                        o[q][e] = base[och[q] * nb[2] + row[q] * nb[1] + xe * nb[0]];
+                    }
+            }
+        };
+        if (a.from_redirect) {
+            float4v o[kGroup];
+            read(a.y, ynb, p.vec_y, o);
+#pragma unroll
+            for (int q = 0; q < kGroup; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) t[q][e] = __fadd_rn(o[q][e], t[q][e]);
+        }
+#pragma unroll 1
+        for (int s = 0; s < a.chain.count; ++s) {
+            const DevStep &st = a.chain.steps[s];
+            if (st.kind == kSilu) {
+#pragma unroll
+                for (int q = 0; q < kGroup; ++q)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) t[q][e] = silu(t[q][e]);
+                continue;
+            }
+            float4v o[kGroup];
+            if (st.nb[0] == 0) {
+                const float *base = st.operand + img * st.nb[3];
+#pragma unroll
+                for (int q = 0; q < kGroup; ++q) {
+                    const float f = base[och[q] * st.nb[2] + row[q] * st.nb[1]];
+                    o[q] = float4v{f, f, f, f};
+                }
+            } else {
+                read(st.operand, st.nb, (p.vec_step >> s) & 1, o);
+            }
+#pragma unroll
+            for (int q = 0; q < kGroup; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    t[q][e] = st.kind == kAdd ? __fadd_rn(t[q][e], o[q][e]) : __fmul_rn(t[q][e], o[q][e]);
+        }
+#pragma unroll
+        for (int q = 0; q < kGroup; ++q) {
+            const int j = KS * (q0 + q) + kg;
+            if (y0 + wp * RW + j / NO >= a.oh || oc0 + 16 * (j % NO) + col >= a.oc || x >= a.ow) continue;
+            float *out = a.y + img * a.ynb3 + och[q] * a.ynb2 + row[q] * a.ynb1 + x;
+            if (p.vec_y) {
+                *reinterpret_cast<float4v *>(out) = t[q];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (x + e < a.ow) out[e] = t[q][e];
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+template <class S>
+__global__ __launch_bounds__(S::kThreads, S::kThreads / 256) void conv3_kernel(Conv3Args p) {
+    constexpr int RW = S::RW, NO = S::NO, KS = S::KS;
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    __shared__ Handover hand;
+    const WinogradArgs &a = p.a;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int steps = (p.chunks + KS - 1) / KS;
+    uint32_t tile = xcd_swizzle(blockIdx.x, gridDim.x);
+    const int count = static_cast<int>((p.tiles - tile + gridDim.x - 1) / gridDim.x);
+    if (wave >= S::kWaves) {
+        fetch_inputs<S>(p, tile, gridDim.x, count, steps, lds, hand);
+        return;
+    }
+    const int wp = wave % S::WP, wo = wave / S::WP % S::WO, kg = wave / (S::WP * S::WO);
+    const int col = lane & 15, quad = lane >> 4;
+
+    // The wave's weights of column kw of a chunk's taps: NO fragments of 16
+    // output channels by the chunk's 32 input channels a tap (channels past the
+    // last read it again).
+    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<_Float16 *>(p.w), 0, static_cast<int>(p.wbytes), 0x00020000);
+    const uint32_t tap_bytes = static_cast<uint32_t>(a.oc) * 64u;
+    half8 wf[2][3][NO];
+    const auto load_w = [&](int set, int oc0, int sc, int kw) {
+        int chunk = sc * KS + kg;
+        chunk = chunk < p.chunks ? chunk : p.chunks - 1;
+        const uint32_t at = static_cast<uint32_t>(chunk * 9 + 3 * kw) * tap_bytes;
+#pragma unroll
+        for (int o = 0; o < NO; ++o) {
+            const int oc = oc0 + 16 * o + col;
+            const uint32_t row = static_cast<uint32_t>(oc < a.oc ? oc : static_cast<int>(a.oc) - 1) * 64u + 16u * quad;
+#pragma unroll
+            for (int kh = 0; kh < 3; ++kh)
+                wf[set][kh][o] = __builtin_bit_cast(
+                    half8, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, row, at + kh * tap_bytes, 0));
+        }
+    };
+    const auto oc_of = [&](int ob) { return ob * S::kOc + wo * 16 * NO; };
+
+    float4v acc[RW][NO];
+    // A chunk's products, its first column's weights in set 0; the next chunk's
+    // are loaded beside its last column and moved there.
+    const auto chunk = [&](const char *buf, bool first, int oc0, int sc, int oc_next, int sc_next) {
+#pragma unroll
+        for (int kw = 0; kw < 3; ++kw) {
+            const int set = kw & 1;
+            if (kw == 1 && first) lds_barrier();  // the fetching waves' (fetch_inputs)
+            half8 x[2][2];
+            const int pos0 = opaque(wp * RW * kPitch + kw + col);  // not thirty addresses held over the chunks
+            const auto read = [&](int r) {
+                const int pos = pos0 + r * kPitch;
+                const char *f = buf + pos * 64 + 16 * (quad ^ ((pos >> 2) & 3));
+                x[r & 1][0] = *reinterpret_cast<const half8 *>(f);
+                x[r & 1][1] = *reinterpret_cast<const half8 *>(f + S::kPlane);
+            };
+            read(0);
+            if (kw < 2) {
+                load_w(set ^ 1, oc0, sc, kw + 1);
+            } else {
+                load_w(set ^ 1, oc_next, sc_next, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < RW + 2; ++r) {
+                if (r + 1 < RW + 2) read(r + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int part = 0; part < 2; ++part)
+#pragma unroll
+                    for (int kh = 0; kh < 3; ++kh) {
+                        if (r - kh < 0 || r - kh >= RW) continue;
+#pragma unroll
+                        for (int o = 0; o < NO; ++o)
+                            acc[r - kh][o] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[r & 1][part], wf[set][kh][o],
+                                                                                   acc[r - kh][o], 0, 0, 0);
+                    }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int kh = 0; kh < 3; ++kh)
+#pragma unroll
+            for (int o = 0; o < NO; ++o) wf[0][kh][o] = wf[1][kh][o];
+    };
+
+    Place at = place_of<S>(p, tile);
+    int oc0 = oc_of(at.ob);
+    load_w(0, oc0, 0, 0);
+    lds_barrier();
+    lds_barrier();
+    int g = 0;
+    for (int left = count; left > 0; --left) {
+        int erun = 0;
+        const Place next = place_of<S>(p, left > 1 ? tile + gridDim.x : tile);
+        const int oc_next = oc_of(next.ob);
+#pragma unroll
+        for (int r = 0; r < RW; ++r)
+#pragma unroll
+            for (int o = 0; o < NO; ++o) acc[r][o] = float4v{};
+        for (int sc = 0; sc < steps; ++sc, ++g) {
+            if (sc > 0) lds_barrier();
+            const int e = __builtin_amdgcn_readfirstlane(hand.e[g & 1]);
+            if (sc > 0 && e != erun) {
+                const float f = ldexpf(1.0f, erun - e);
+#pragma unroll
+                for (int r = 0; r < RW; ++r)
+#pragma unroll
+                    for (int o = 0; o < NO; ++o) acc[r][o] *= f;
+            }
+            erun = e;
+            const char *buf = lds + (g & 1) * S::kBuffer + kg * 2 * S::kPlane;
+            const bool last = sc + 1 == steps;
+            chunk(buf, g == 0, oc0, sc, last ? oc_next : oc0, last ? 0 : sc + 1);
+        }
+        finish<S>(p, at, oc0, wp, wo, kg, wave, lane, erun, acc, lds);
+        lds_barrier();
+        tile += gridDim.x;
+        at = next;
+        oc0 = oc_next;
+    }
+}
+
+// ------------------------------------------------------------------ host
+
+template <class S>
+int64_t blocks_of(const WinogradArgs &a) {
+    return ceil_div(a.ow, kCols) * ceil_div(a.oh, S::kRows) * a.n * ceil_div(a.oc, S::kOc);
+}
+
+// What a form takes on one CU, in thousands of cycles (timestamps of the three
+// kernels): a step of the input channels, and a tile's beginning and end.
+struct Cost {
+    double step, tile;
+};
+
+template <class S>
+double cycles_of(const WinogradArgs &a, Cost c) {
+    const int64_t rounds = ceil_div(blocks_of<S>(a), compute_units());
+    return static_cast<double>(rounds) * (static_cast<double>(ceil_div(a.ic, kChunk * S::KS)) * c.step + c.tile) + 12.0;
+}
+
+// The form of the least cycles: 1 Wide, 2 Mid, 3 Narrow.
+int shape_of(const WinogradArgs &a, double &cycles) {
+    const double c[3] = {cycles_of<Wide>(a, {11.4, 26.0}), cycles_of<Mid>(a, {8.5, 14.0}),
+                         cycles_of<Narrow>(a, {9.7, 14.0})};
+    int best = 0;
+    for (int i = 1; i < 3; ++i)
+        if (c[i] < c[best]) best = i;
+    cycles = c[best];
+    return best + 1;
+}
+
+// Whether the products here take less than F(4x4)'s launches: microseconds of
+// both, fitted to measurements.  Here: the cycles at 2.3 GHz and the pass over
+// the weights.  There: the bytes of its four passes (18 an input, 22 an output,
+// 150 a kernel), its products at the rate the MFMA reaches there, its launches;
+// or, on few tiles, the small images' path, which its kernels bound.
+// Measured, here and F(4x4), us (2 images of a UNet level, 1 of the VAE's):
+//   320->320 64x64   40.4   48.8    128->128 520x768  286   595
+//   1280->640 32x32  71.7  105.1    256->256 256x256  150   217
+//   640->640 33x48   56.3   64.6    512->512 128x128  130   138
+//   1280->1280 16x16 68.2   73.9    512->512 67x117   109   107
+//   2560->1280 16x16  126    116    960->640 45x33    145   111
+bool direct_faster(const WinogradArgs &a) {
+    double cycles = 0.0;
+    shape_of(a, cycles);
+    const double kernels = static_cast<double>(a.ic * a.oc);
+    const double in = static_cast<double>(a.n * a.ic * a.ih * a.iw), out = static_cast<double>(a.n * a.oc * a.oh * a.ow);
+    const double here = 6.0 + cycles / 2.3 + 36.0 * kernels / 4.5e6;
+    const double there =
+        a.tiles <= 32 ? 32.0 + 25.0 * kernels / 1e6
+                      : 16.0 + (18.0 * in + 22.0 * out + 150.0 * kernels) / 4.5e6 + 0.75 * 18.0 * out * a.ic / 1.1e9;
+    return here <= there;
+}
+
+int64_t weight_bytes(const WinogradArgs &a) { return a.ic * a.oc * 18; }
+
+// An image's floats from its first past its last.
+int64_t image_floats(const WinogradArgs &a) { return (a.ic - 1) * a.xnb2 + (a.ih - 1) * a.xnb1 + a.iw; }
+
+template <class S>
+hipError_t launch(Conv3Args &p, hipStream_t stream) {
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&conv3_kernel<S>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds);
+    if (attr != hipSuccess) return attr;
+    p.tiles_x = static_cast<int32_t>(ceil_div(p.a.ow, kCols));
+    p.tiles_y = static_cast<int32_t>(ceil_div(p.a.oh, S::kRows));
+    p.tiles = static_cast<uint32_t>(blocks_of<S>(p.a));
+    // A workgroup a CU, tile after tile, where one holds all the input
+    // channels' groups; else one a tile.
+    const uint32_t cus = static_cast<uint32_t>(compute_units());
+    const uint32_t blocks = S::KS == 1 && p.tiles > cus ? cus : p.tiles;
+    SDHIP_LAUNCH(conv3_kernel<S>, dim3(blocks), dim3(S::kThreads), S::kLds, stream, p);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+bool conv3_shape(const WinogradArgs &a) {
+    const Tuning &t = tuning();
+    if (a.m != 4 || a.w32 != nullptr || t.winograd_fp32 || t.gemm_core != 0 || t.gemm_tiles != 0) return false;
+    if (a.ic % kChunk != 0 || a.ic < 128 || a.oc < 128) return false;
+    if (a.xnb1 < a.iw || a.xnb2 < 1 || a.xnb3 < 0 || a.n < 1) return false;
+    // Offsets in an image, in the weights and of blocks in 31 bits.
+    if (image_floats(a) * 4 >= (int64_t{1} << 31) - 64 || weight_bytes(a) >= (int64_t{1} << 31) - 64) return false;
+    return blocks_of<Narrow>(a) < (int64_t{1} << 22) && direct_faster(a);
+}
+
+// One pass reads the inputs while it writes the outputs: not in place.
+bool conv3_taken(const WinogradArgs &a) {
+    if (!conv3_shape(a)) return false;
+    const int64_t x_floats = (a.n - 1) * a.xnb3 + image_floats(a);
+    const int64_t y_floats = (a.n - 1) * a.ynb3 + (a.oc - 1) * a.ynb2 + (a.oh - 1) * a.ynb1 + a.ow;
+    return !spans_overlap(a.x, static_cast<size_t>(x_floats) * 4, a.y, static_cast<size_t>(y_floats) * 4);
+}
+
+size_t conv3_work_size(const WinogradArgs &a) { return static_cast<size_t>(round_up(weight_bytes(a), 256)); }
+
+sdhip_status conv3(const WinogradArgs &a, void *work, hipStream_t stream) {
+    Conv3Args p{};
+    p.a = a;
+    p.chunks = static_cast<int32_t>(a.ic / kChunk);
+    p.xbytes = static_cast<uint32_t>(image_floats(a) * 4);
+    p.wbytes = static_cast<uint32_t>(weight_bytes(a));
+    const auto quads = [](const float *t, int64_t nb1, int64_t nb2, int64_t nb3) {
+        return (reinterpret_cast<uintptr_t>(t) & 15) == 0 && nb1 % 4 == 0 && nb2 % 4 == 0 && nb3 % 4 == 0;
+    };
+    p.vec_y = a.ow % 4 == 0 && quads(a.y, a.ynb1, a.ynb2, a.ynb3);
+    for (int s = 0; s < a.chain.count; ++s) {
+        const DevStep &st = a.chain.steps[s];
+        if (st.kind != kSilu && a.ow % 4 == 0 && st.nb[0] == 1 && quads(st.operand, st.nb[1], st.nb[2], st.nb[3]))
+            p.vec_step |= 1u << s;
+    }
+    // The weights in the products' order, kept in the store when it has room,
+    // as Winograd's transformed ones are.
+    const int64_t wne[4] = {3, 3, a.ic, a.oc};
+    const int64_t wnb[4] = {2, 6, 18, 18 * a.ic};
+    bool ready = false;
+    void *kept = store_entry(a.w, SDHIP_TYPE_F16, wne, wnb, kStoreConv3, 0, static_cast<size_t>(weight_bytes(a)),
+                             static_cast<size_t>(weight_bytes(a)), stream, ready);
+    _Float16 *wt = static_cast<_Float16 *>(kept != nullptr ? kept : work);
+    p.w = wt;
+    if (!ready) {
+        KernelScope scope("conv3x3.weights", stream);
+        SDHIP_LAUNCH(conv3_weights_kernel,
+                     dim3(static_cast<uint32_t>(p.chunks), static_cast<uint32_t>(ceil_div(a.oc, 8))), dim3(256), 0, stream,
+                     a.w, a.oc, a.ic, wt);
+        const hipError_t err = hipGetLastError();
+        if (err != hipSuccess) return launched(err, "conv2d weights");
+        if (kept != nullptr) store_publish(kept);
+    }
+    KernelScope scope("conv3x3.products", stream);
+    double cycles = 0.0;
+    const int shape = shape_of(a, cycles);
+    const hipError_t err = shape == 1 ? launch<Wide>(p, stream) : shape == 2 ? launch<Mid>(p, stream) : launch<Narrow>(p, stream);
+    return launched(err, "conv2d 3x3");
+}
+
+}  // namespace sdhip

@@ -6,7 +6,9 @@
 // F(2x2, 3x3) with the matrices of winograd.cc:19-22 and F(4x4, 3x3) with the
 // points 0, 1, -1, 2, -1/2, infinity of winograd.cc:1146-1183, 1259-1264.
 //
-// On the device, in five launches:
+// FP16 kernels of 128 channels and more whose F(4x4) would spend its time on the
+// bytes between its launches are computed directly instead (conv3.hip).  On the
+// device, in five launches:
 //   0. the scales, exact powers of two: each input channel's e_c, its
 //      greatest |x| times the input transform's gain (49 for F(4x4), 4 for
 //      F(2x2)) below 2^(17 + e_c); each output channel's a_o, its greatest
@@ -38,6 +40,7 @@
 // With winograd_fp32=1 the products go to the single-precision MFMA instead
 // (v_mfma_f32_16x16x4_f32), unscaled: a sixteenth of the rate, for comparison.
 
+#include "conv3.h"
 #include "host.h"
 #include "kernels.h"
 #include "profile.h"
@@ -1556,9 +1559,16 @@ sdhip_status run(const WinogradArgs &in, void *work, hipStream_t stream) {
 
 }  // namespace
 
-size_t winograd_work_size(const WinogradArgs &a) { return work_layout(a).total; }
+// Either form's: which of the two a call takes depends on where its operands
+// lie, which the query of the size may not know.
+size_t winograd_work_size(const WinogradArgs &a) {
+    const size_t winograd = work_layout(a).total, direct = conv3_shape(a) ? conv3_work_size(a) : 0;
+    return direct > winograd ? direct : winograd;
+}
 
 sdhip_status winograd(const WinogradArgs &a, void *work, hipStream_t stream) {
+    // Directly where that is the faster (conv3.hip).
+    if (conv3_taken(a)) return conv3(a, work, stream);
     return a.m == 4 ? run<4>(a, work, stream) : run<2>(a, work, stream);
 }
 

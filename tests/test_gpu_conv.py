@@ -423,3 +423,92 @@ def test_conv_panels(gpu, c, form):
         assert err <= BOUND
         outs.append(got)
     assert orc.metric(outs[0], outs[1], m2) <= BOUND
+
+
+def kernel_names(fn):
+    sdhip.profile_reset()
+    sdhip.profile_enable(True)
+    try:
+        fn()
+        torch.cuda.synchronize()
+        return set(sdhip.profile_collect())
+    finally:
+        sdhip.profile_enable(False)
+
+
+CONV3_CASES = [  # n, ic, oc, h, w, padding: 3x3 convolutions taken directly, by the three forms
+    (1, 128, 128, 261, 303, 1),  # several tiles a workgroup, ragged rows and columns, scalar stores
+    (1, 128, 200, 250, 320, 2),  # channels past OC, a border of 2
+    (2, 320, 320, 64, 64, 1),    # 64 by 160
+    (2, 160, 320, 62, 64, 1),    # a chunk short of the last pair
+    (2, 640, 640, 34, 34, 0),    # 64 by 80, groups of four chunks, no border
+    (2, 416, 600, 32, 32, 1),    # the same, chunks short of the last four, channels past OC
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", CONV3_CASES, ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("form", ["bias_scale_silu_residual", "from_redirect", "strided", "range"])
+def test_conv3_direct(gpu, c, form):
+    """Against float64 by the reference's metric: 22 bits of each input and
+    single-precision sums stay within 2e-6 (the bound of the operation is
+    2e-5); `strided` a view of a larger input and a transposed residual;
+    `range` inputs whose channels and rows lie 2^-30 .. 2^30 apart, so that
+    the tiles' scales differ and move."""
+    n, ic, oc, h, w, p = c
+    g = torch.Generator(device="cpu").manual_seed(n + ic + oc + h + w)
+    x = torch.randn((n, ic, h, w), generator=g)
+    if form == "range":
+        x *= torch.exp2(torch.randint(-30, 31, (1, ic, 1, 1), generator=g).float())
+        x *= torch.exp2(torch.randint(-6, 7, (1, 1, h, 1), generator=g).float())
+    k = (0.05 * torch.randn((oc, ic, 3, 3), generator=g)).half()
+    oh, ow = h + 2 * p - 2, w + 2 * p - 2
+    want = torch.nn.functional.conv2d(x.double(), k.double(), padding=p)
+    mag = torch.nn.functional.conv2d(x.double().abs(), k.double().abs(), padding=p)
+    x_d, k_d = x.to(gpu), k.to(gpu)
+    if form == "strided":
+        wide = torch.full((n, ic, h + 3, w + 5), float("nan"), device=gpu)
+        wide[:, :, 1:h + 1, 2:w + 2] = x_d
+        x_d = wide[:, :, 1:h + 1, 2:w + 2]
+    y = torch.full((n, oc, oh, ow), float("nan"), device=gpu)
+    bias, scale = torch.randn((1, oc, 1, 1), generator=g), torch.randn((n, oc, 1, 1), generator=g)
+    residual = torch.randn((n, oc, oh, ow), generator=g)
+    chain = None
+    out = y
+    if form == "bias_scale_silu_residual":
+        chain = sdhip.epilogue([("add", bias.to(gpu)), ("mul", scale.to(gpu)), ("silu", None), ("add", residual.to(gpu))])
+        want = torch.nn.functional.silu((want + bias) * scale) + residual
+        mag = (mag + bias.abs()) * scale.abs() + residual.abs()
+    elif form == "strided":
+        turned = residual.transpose(2, 3).contiguous().to(gpu).transpose(2, 3)  # x not its contiguous dimension
+        with pytest.raises(sdhip.SdhipError):
+            sdhip.conv2d(k_d, x_d, y, sdhip.conv_params(1, 1, p, p, 1, 1), sdhip.epilogue([("add", turned)]))
+        chain = sdhip.epilogue([("add", residual[:, :, :, :1].contiguous().to(gpu))])
+        want, mag = want + residual[:, :, :, :1], mag + residual[:, :, :, :1].abs()
+    elif form == "from_redirect":
+        out = residual.to(gpu)
+        chain = sdhip.epilogue([("add", bias.to(gpu))], redirect=out, from_redirect=True)
+        want, mag = want + residual + bias, mag + residual.abs() + bias.abs()
+    names = kernel_names(lambda: sdhip.conv2d(k_d, x_d, y, sdhip.conv_params(1, 1, p, p, 1, 1), chain))
+    assert "conv3x3.products" in names
+    got = out.cpu().double()
+    assert torch.isfinite(got).all()
+    err = ((got - want).abs() / mag.clamp_min(1e-300)).max().item()
+    print(f"conv3 {c} {form}: {err:.3g}")
+    assert err <= 2e-6
+
+
+@pytest.mark.gpu
+def test_conv3_in_place_takes_winograd(gpu):
+    """A convolution whose residual connection is written over its own inputs
+    reads them all before it writes: not taken in one pass."""
+    g = torch.Generator(device="cpu").manual_seed(3)
+    x, k = torch.randn((2, 320, 64, 64), generator=g), (0.02 * torch.randn((320, 320, 3, 3), generator=g)).half()
+    x_d, k_d = x.to(gpu), k.to(gpu)
+    y = torch.empty_like(x_d)
+    names = kernel_names(lambda: sdhip.conv2d(k_d, x_d, y, sdhip.conv_params(1, 1, 1, 1, 1, 1),
+                                              sdhip.epilogue([], redirect=x_d, from_redirect=True)))
+    assert "winograd4.products" in names
+    want = torch.nn.functional.conv2d(x.double(), k.double(), padding=1) + x
+    mag = torch.nn.functional.conv2d(x.double().abs(), k.double().abs(), padding=1) + x.abs()
+    assert ((x_d.cpu().double() - want).abs() / mag).max().item() <= BOUND
