@@ -16,7 +16,7 @@ struct GroupNormArgs {
     int64_t xnb2, xnb3, ynb2, ynb3;
     int64_t groups, per_group;
     int64_t chunk, slices;  // numbers of a slice; slices of a group
-    double *partials;       // [2][ne3 * groups][slices]: sums of x, then of (x - mean)^2
+    double *partials;       // [2][ne3 * groups][slices]: sums of x, then of (x - the slice's mean)^2
     float eps;
     DevChain chain;
 };

@@ -3,10 +3,12 @@
 // sum in double precision; the variance as float(sum((x - mean)^2) / n), each
 // difference and square in single precision and the sum in double; the scale
 // 1 / sqrt(variance + eps) in single precision, correctly rounded; the output
-// (x - mean) * scale and then the chain (norm.cc:44-175).  Only the order of
-// the double-precision sums differs from the reference's eight lanes.
+// (x - mean) * scale and then the chain (norm.cc:44-175).  The order of the
+// double-precision sums differs from the reference's eight lanes; and a group of
+// several slices takes its squares about each slice's mean first (below).
 
 #include <mutex>
+#include <type_traits>
 
 #include "host.h"
 #include "norm.h"
@@ -24,13 +26,16 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// GROUP_NORM in three launches over blocks of (image, group, slice), the
-// slices `chunk` consecutive numbers of the group's channels (consecutive
-// planes, ne0 * ne1 numbers each): the partial sums of x; from their total
-// the mean, and the partial sums of (x - mean)^2; from both totals the scale,
-// and the output with its chain.  Each sum of a slice goes to the work buffer
-// and is added up, in the order of the slices, by each block that needs the
-// total.
+// GROUP_NORM in two launches over blocks of (image, group, slice), the slices
+// `chunk` consecutive numbers of the group's channels (consecutive planes, ne0
+// * ne1 numbers each): each slice's sum S of x and sum of (x - m)^2, m the
+// slice's own mean in single precision; then, from all of a group's,
+//     sum (x - mean)^2 = sum over slices of [sum (x - m)^2 + 2 (m - mean) (S - n m)
+//                        + n (m - mean)^2]
+// in double, the scale, and the output with its chain.  A pass over the group's
+// mean first took a third launch (4.2 us of 33 for 1280 channels of 32 x 32, two
+// images, after their convolution); a slice's numbers stay in registers between
+// its two sums, or are read again from L2 where they are more than those hold.
 
 struct GroupView {
     int64_t item, slice, i3, c0, count, e0, e1;
@@ -61,13 +66,6 @@ __device__ __forceinline__ double block_sum(double v, double *lds_sums) {
     return s;
 }
 
-// The total over the slices of an item, in their order.
-__device__ __forceinline__ double total(const double *partials, int64_t item, int64_t slices) {
-    double t = 0.0;
-    for (int64_t q = 0; q < slices; ++q) t += partials[item * slices + q];
-    return t;
-}
-
 // PASS 0: the sum of x over the block's slice; PASS 1: of (x - mean)^2, each
 // difference and square in single precision (norm.cc:44-90).
 template <int PASS>
@@ -77,24 +75,14 @@ __device__ __forceinline__ double term(float x, float mean) {
     return static_cast<double>(__fmul_rn(d, d));
 }
 
+// The sum of the slice's terms, x from the group's first number, `quads` where it
+// is 16-byte aligned.
 template <int PASS>
-__global__ __launch_bounds__(kThreads) void group_sums_kernel(GroupNormArgs a) {
-    __shared__ double lds_sums[kThreads / 64];
-    __shared__ float shared_mean;
-    const GroupView g = group_view(a);
+__device__ __forceinline__ double slice_terms(const GroupView &g, const float *x, bool quads, float mean) {
     const int tid = threadIdx.x;
-    float mean = 0.0f;
-    if (PASS == 1) {
-        if (tid == 0 && g.count > 0) {
-            shared_mean = static_cast<float>(total(a.partials, g.item, a.slices) / static_cast<double>(g.count));
-        }
-        __syncthreads();
-        mean = shared_mean;
-    }
-    const float *x = a.x + g.i3 * a.xnb3 + g.c0 * a.xnb2;
     double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    if ((reinterpret_cast<uintptr_t>(x) & 15) == 0) {
-        // a.chunk is a multiple of 4: the slice's quads start at e0 / 4.
+    if (quads) {
+        // The chunk is a multiple of 4: the slice's quads start at e0 / 4.
         const float4 *x4 = reinterpret_cast<const float4 *>(x);
         const int64_t q1 = g.e1 / 4;
         int64_t i = g.e0 / 4 + tid;
@@ -113,8 +101,73 @@ __global__ __launch_bounds__(kThreads) void group_sums_kernel(GroupNormArgs a) {
     } else {
         for (int64_t e = g.e0 + tid; e < g.e1; e += kThreads) s0 += term<PASS>(x[e], mean);
     }
-    const double sum = block_sum((s0 + s1) + (s2 + s3), lds_sums);
-    if (tid == 0) a.partials[(PASS * a.ne3 * a.groups + g.item) * a.slices + g.slice] = sum;
+    return (s0 + s1) + (s2 + s3);
+}
+
+// A slice's own mean, as both launches take it.
+__device__ __forceinline__ float slice_mean(double sum, int64_t n) {
+    return n > 0 ? static_cast<float>(sum / static_cast<double>(n)) : 0.0f;
+}
+
+constexpr int kStatQuads = 4;  // float4 of a slice a thread holds
+
+__global__ __launch_bounds__(kThreads) void group_stats_kernel(GroupNormArgs a) {
+    __shared__ double lds_sums[kThreads / 64];
+    const GroupView g = group_view(a);
+    const int tid = threadIdx.x;
+    const float *x = a.x + g.i3 * a.xnb3 + g.c0 * a.xnb2;
+    const bool quads = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+    double sum, squares;
+    if (quads && a.chunk <= 4 * kStatQuads * kThreads && g.e1 % 4 == 0) {
+        const float4v *x4 = reinterpret_cast<const float4v *>(x);
+        float4v v[kStatQuads];
+        bool in[kStatQuads];
+#pragma unroll
+        for (int u = 0; u < kStatQuads; ++u) {
+            const int64_t i = g.e0 / 4 + tid + kThreads * u;
+            in[u] = i < g.e1 / 4;
+            v[u] = in[u] ? x4[i] : float4v{};
+        }
+        const auto over = [&](auto pass, float mean) {
+            double s = 0.0;
+#pragma unroll
+            for (int u = 0; u < kStatQuads; ++u) {
+                if (!in[u]) continue;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) s += term<decltype(pass)::value>(v[u][k], mean);
+            }
+            return block_sum(s, lds_sums);
+        };
+        sum = over(std::integral_constant<int, 0>{}, 0.0f);
+        squares = over(std::integral_constant<int, 1>{}, slice_mean(sum, g.e1 - g.e0));
+    } else {
+        sum = block_sum(slice_terms<0>(g, x, quads, 0.0f), lds_sums);
+        squares = block_sum(slice_terms<1>(g, x, quads, slice_mean(sum, g.e1 - g.e0)), lds_sums);
+    }
+    if (tid == 0) {
+        a.partials[g.item * a.slices + g.slice] = sum;
+        a.partials[(a.ne3 * a.groups + g.item) * a.slices + g.slice] = squares;
+    }
+}
+
+// A group's mean and scale from its slices' sums, by a wave.
+__device__ __forceinline__ void group_stats(const GroupNormArgs &a, const GroupView &g, float &mean, float &scale) {
+    const int lane = threadIdx.x & 63;
+    const double *sums = a.partials + g.item * a.slices;
+    const double *squares = sums + a.ne3 * a.groups * a.slices;
+    const double n = static_cast<double>(g.count);
+    double t = 0.0;
+    for (int64_t q = lane; q < a.slices; q += 64) t += sums[q];
+    mean = static_cast<float>(wave_sum(t) / n);
+    t = 0.0;
+    for (int64_t q = lane; q < a.slices; q += 64) {
+        const int64_t e0 = q * a.chunk, e1 = e0 + a.chunk < g.count ? e0 + a.chunk : g.count;
+        const int64_t len = e1 > e0 ? e1 - e0 : 0;
+        const double m = slice_mean(sums[q], len), d = m - mean, ln = static_cast<double>(len);
+        t += squares[q] + d * (2.0 * (sums[q] - ln * m) + ln * d);
+    }
+    const float variance = static_cast<float>(wave_sum(t) / n);
+    scale = __fdiv_rn(1.0f, __fsqrt_rn(variance + a.eps));
 }
 
 // The most channels a slice's operands of one number a channel are held
@@ -128,13 +181,13 @@ __global__ __launch_bounds__(kThreads) void group_apply_kernel(GroupNormArgs a) 
     __shared__ float shared[2];
     const GroupView g = group_view(a);
     const int tid = threadIdx.x;
-    if (tid == 0 && g.count > 0) {
-        const double n = static_cast<double>(g.count);
-        const float mean = static_cast<float>(total(a.partials, g.item, a.slices) / n);
-        const float variance =
-            static_cast<float>(total(a.partials + a.ne3 * a.groups * a.slices, g.item, a.slices) / n);
-        shared[0] = mean;
-        shared[1] = __fdiv_rn(1.0f, __fsqrt_rn(variance + a.eps));
+    if (tid < 64 && g.count > 0) {
+        float mean, scale;
+        group_stats(a, g, mean, scale);
+        if (tid == 0) {
+            shared[0] = mean;
+            shared[1] = scale;
+        }
     }
     __syncthreads();
     const float mean = shared[0], scale = shared[1];
@@ -260,7 +313,7 @@ __global__ __launch_bounds__(kThreads) void group_apply_kernel(GroupNormArgs a) 
 // GROUP_NORM of small groups in one launch: a block of 1024 threads per
 // (image, group) holds the group's count <= kResident numbers in registers,
 // four consecutive numbers of one channel a thread at a time (planes of a
-// multiple of 4), and takes the same statistics as the three launches above
+// multiple of 4), and takes the statistics the two launches above come to
 // -- float(sum / n) with the sum in double, then float(sum of the single-
 // precision squares of x - mean / n) -- with x read once.
 constexpr int kResidentThreads = 1024;
@@ -572,12 +625,8 @@ hipError_t launch_group_norm(const GroupNormArgs &a, hipStream_t stream) {
     }
     const dim3 grid(static_cast<uint32_t>(a.ne3 * a.groups * a.slices));
     {
-        KernelScope scope("group_norm.sums", stream);
-        SDHIP_LAUNCH(group_sums_kernel<0>, grid, dim3(kThreads), 0, stream, a);
-    }
-    {
-        KernelScope scope("group_norm.squares", stream);
-        SDHIP_LAUNCH(group_sums_kernel<1>, grid, dim3(kThreads), 0, stream, a);
+        KernelScope scope("group_norm.stats", stream);
+        SDHIP_LAUNCH(group_stats_kernel, grid, dim3(kThreads), 0, stream, a);
     }
     KernelScope scope("group_norm.apply", stream);
     SDHIP_LAUNCH(group_apply_kernel, grid, dim3(kThreads), 0, stream, a);

@@ -124,3 +124,30 @@ def test_norm_rows_and_operands(gpu, shape, view):
     diff = np.abs(got - want).max() / np.abs(want).max()
     print(f"norm {shape} view={view}: {diff:.3g} of the largest")
     assert diff <= CLOSE
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,groups,offset", [
+    ((1, 32, 256, 256), 1, 0),     # one group: more slices than a wave has lanes
+    ((2, 34, 65, 67), 2, 0),       # planes of no multiple of 4, the last slice short
+    ((1, 48, 64, 64), 3, 1),       # rows that start between quads
+    ((1, 4, 512, 512), 2, 0),      # slices read twice
+])
+def test_group_norm_slices(gpu, shape, groups, offset):
+    """Groups of several slices whose means differ by hundreds of their
+    deviations: the squares about each slice's own mean, put together, against
+    float64.  A number of 1000 is rounded by 3e-5 in single precision and the
+    mean likewise; over the group's deviation, about 300, that is 2e-7."""
+    r = rng(sum(shape) + groups)
+    n = int(np.prod(shape))
+    x = (np.linspace(-500.0, 500.0, n) + r.standard_normal(n)).astype(np.float32).reshape(shape)
+    flat = torch.empty(n + 4, device=gpu)
+    x_d = flat[offset:offset + n].view(shape)
+    x_d.copy_(torch.from_numpy(x))
+    y = unwritten(shape, gpu)
+    sdhip.group_norm(x_d, y, groups, 1e-5)
+    torch.cuda.synchronize()
+    want = torch.nn.functional.group_norm(torch.from_numpy(x).double(), groups, eps=1e-5).numpy()
+    diff = np.abs(y.cpu().numpy() - want).max()
+    print(f"group_norm slices {shape}/{groups}: {diff:.3g}")
+    assert diff <= 1e-6
