@@ -1809,13 +1809,16 @@ hipError_t launch_few(const AttentionArgs &a, hipStream_t stream) {
     // each about as many.  Workgroups of eight waves, or of four where those
     // would leave half the CUs without one (1024 queries of 16 heads of 80, 64
     // workgroups of eight: 12.9 us, of four 11.9; 988 of 40 heads of 64, 160 of
-    // eight: 13.0, of four 19.1).
+    // eight: 13.0, of four 19.1), or where a grid of eight, one dimension of
+    // under 2^32 threads, would not hold the heads.
     const int64_t wave_tiles = ceil_div(a.lq, 32);
-    const int64_t waves = F::kWaves == 8 && 2 * heads * ceil_div(wave_tiles, 8) >= compute_units() ? 8 : 4;
+    const bool eight = F::kWaves == 8 && heads < (int64_t{1} << 23) &&
+                       2 * heads * ceil_div(wave_tiles, 8) >= compute_units();
+    const int64_t waves = eight ? 8 : 4;
     const int64_t most = 8 * compute_units() / heads > waves ? 8 * compute_units() / heads : waves;
     const int64_t rounds = ceil_div(wave_tiles, most);
     const int64_t per_head = ceil_div(ceil_div(wave_tiles, rounds), waves);
-    if (heads * per_head >= (int64_t{1} << 22)) return hipErrorInvalidValue;
+    if (heads * per_head * 64 * waves >= (int64_t{1} << 32)) return hipErrorInvalidValue;
     KernelScope scope("attention", stream);
     SDHIP_LAUNCH(attention_few_kernel<D>, dim3(static_cast<uint32_t>(heads * per_head)), dim3(static_cast<uint32_t>(64 * waves)), lds,
                  stream, a, static_cast<uint32_t>(per_head));

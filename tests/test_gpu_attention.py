@@ -337,3 +337,18 @@ def test_attention_few_keys(gpu, d, lq, lk, h, hk, b):
     print(f"few keys {(d, lq, lk, h, hk, b)}: {err:.3g}")
     assert np.isfinite(y).all()
     assert err <= BOUND
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads", [2 ** 22 + 1, 2 ** 23 + 1])
+def test_attention_few_keys_many_heads(gpu, heads):
+    """One query and one key of more heads than workgroups of eight waves fill
+    half a grid, or all of one: every output is the value, of which two FP16
+    parts hold 22 bits (and the sum's reciprocal rounds once more: 2^-21)."""
+    q = torch.ones((1, 1, heads, 32), device=gpu)
+    k, v = torch.randn((2, 1, 1, 1, 32), generator=torch.Generator().manual_seed(7)).to(gpu)
+    y = unwritten((1, 1, heads, 32), gpu)
+    sdhip.attention(*(t.permute(0, 2, 1, 3) for t in (q, k, v)), y, 1.0)
+    torch.cuda.synchronize()
+    # Numbers under 2^-6 are 2^-31 off at most (an FP16 subnormal of the second part, taken 2^-4 times).
+    assert ((y - v).abs() <= v.abs() * 2.0 ** -21 + 2.0 ** -30).all()
