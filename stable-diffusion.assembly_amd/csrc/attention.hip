@@ -431,13 +431,13 @@ __global__ __launch_bounds__(256) void attention_wide_kernel(AttentionArgs a, in
 }
 
 // Heads of up to 512 dimensions (more than 384) with single-precision keys
-// and values, where attention512.hip does not take them (fewer positions,
-// rows not 16-byte aligned, or attention_fp32=1): the wide form's products, softmax and sums, in the same
-// order -- bit for bit its output -- with each wave's 16 queries held in
-// registers for the whole split (lane (lr, lg) holds dimensions 4 j + lg of
-// query lr: operand B of step j) and a block's 32 keys and their values
-// staged whole in LDS, rows of DP + 4 and 16 NDV + 4 floats (64 banks for
-// both reads), float4 copies: two barriers a block of keys, where the wide
+// and values, where attention512.hip does not take them (fewer positions, rows
+// not 16-byte aligned, or attention_fp32=1): the wide form's products, softmax
+// and sums, in the same order -- bit for bit its output -- with each wave's 16
+// queries held in registers for the whole split (lane (lr, lg) holds dimensions
+// 4 j + lg of query lr: operand B of step j) and a block's 32 keys and their
+// values staged whole in LDS, rows of DP + 4 and 16 NDV + 4 floats (64 banks
+// for both reads), float4 copies: two barriers a block of keys, where the wide
 // form restages its queries with every chunk of every block.
 template <int DP, int NDV>
 __global__ __launch_bounds__(256, 1) void attention_wide2_kernel(AttentionArgs a, int64_t splits, int64_t key_len,
@@ -1496,13 +1496,13 @@ __global__ __launch_bounds__(256, OCC) void attention_split_kernel(AttentionArgs
 // What bounds it: HBM and the first wait (4 .. 5 us of load, split and
 // barrier).  A workgroup of its own for every 128 queries, which splits the
 // keys and values each time, took 25.9 us for 6240 queries of 16 heads of 40
-// and 77 keys (32 MB, 6.3 us at a copy's rate); this form 16.1, of which a wave's
+// and 77 keys (32 MB, 6.3 us at a copy's rate); this form 15.6, of which a wave's
 // second 32 queries are about 5 (a chain of products, maximum, exponentials and
 // products with one other wave on the SIMD beside it).  Tiles of 64 and 96 keys,
 // for longer chains side by side: 20.3 and 23.3 us (registers spilled).
 template <int D>
 struct Few {
-    static constexpr int kKeys = D <= 64 ? 32 : 32;  // a tile's
+    static constexpr int kKeys = 32;                  // a tile's
     static constexpr int kWaves = D <= 96 ? 8 : 4;    // the most waves of a workgroup
     static constexpr bool kAhead = D <= 80;  // the next queries' rows loaded ahead, where the registers allow it
     static constexpr int kRecord = Split<D, kKeys>::kRecord;
@@ -1820,8 +1820,8 @@ hipError_t launch_few(const AttentionArgs &a, hipStream_t stream) {
     const int64_t per_head = ceil_div(ceil_div(wave_tiles, rounds), waves);
     if (heads * per_head * 64 * waves >= (int64_t{1} << 32)) return hipErrorInvalidValue;
     KernelScope scope("attention", stream);
-    SDHIP_LAUNCH(attention_few_kernel<D>, dim3(static_cast<uint32_t>(heads * per_head)), dim3(static_cast<uint32_t>(64 * waves)), lds,
-                 stream, a, static_cast<uint32_t>(per_head));
+    SDHIP_LAUNCH(attention_few_kernel<D>, dim3(static_cast<uint32_t>(heads * per_head)),
+                 dim3(static_cast<uint32_t>(64 * waves)), lds, stream, a, static_cast<uint32_t>(per_head));
     return hipGetLastError();
 }
 
