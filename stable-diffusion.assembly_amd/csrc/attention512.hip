@@ -37,10 +37,10 @@
 // between them the waves of a SIMD wait together for the softmax and its three
 // barriers, about 2900.  Halving the loads changed 3%.  One head of 512 over
 // 4096 positions: 793 -> 130 us a pass (traced one by one: the products 678 ->
-// 123, the merge of half as many splits 46 -> 10, the tiles 12), error against 64 bits 9.0e-7
-// -> 4.4e-7; 1024 positions 163 -> 44 us.  Slower: the next step's scores
-// beside the softmax or after the outputs with no barrier between (132 and 149
-// us for the kernel, the registers spilled).
+// 123, the merge of half as many splits 46 -> 10, the tiles 12), error against
+// 64 bits 9.0e-7 -> 4.4e-7; 1024 positions 163 -> 44 us.  Slower: the next
+// step's scores beside the softmax or after the outputs with no barrier between
+// (132 and 149 us for the kernel, the registers spilled).
 
 #include "attention.h"
 #include "host.h"
