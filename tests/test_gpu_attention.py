@@ -314,6 +314,88 @@ def test_attention512(gpu, c, spread):
     assert errors[""] <= 1.5 * errors["attention_fp32=1"] + 1e-7
 
 
+def attention512_case(gpu, q, k, v):
+    """The default form's and the single-precision form's errors (attention_fp32=1)
+    against float64 by the reference's metric."""
+    b, lq, h, d = q.shape
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(d)))
+    exact, mag = orc.exact_attention(q, k, v, scale)
+    views = [dev(t, gpu).permute(0, 2, 1, 3) for t in (q, k, v)]
+    errors = []
+    for tuning in ("", "attention_fp32=1"):
+        y = unwritten((b, lq, h, v.shape[3]), gpu)
+        sdhip.set_tuning(tuning)
+        try:
+            sdhip.attention(*views, y, scale)
+        finally:
+            sdhip.set_tuning("")
+        torch.cuda.synchronize()
+        errors.append(orc.metric(y.cpu().numpy(), exact, mag))
+    return errors
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [(512, 1024, 1024, 1, 1, 1), (400, 1000, 1027, 2, 1, 1), (512, 16384, 40, 1, 1, 1),
+                               (388, 16380, 7, 1, 1, 1)], ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("form", ["weightless key", "value dimensions", "query dimensions", "within the split"])
+def test_attention512_far_apart(gpu, c, form):
+    """Numbers that two FP16 parts beside one scale do not hold: a key without
+    weight (its score 60 below the others, in base 2) whose values are 2^20
+    times the others'; values' dimensions 2^-16 .. 2^16 apart; queries'
+    dimensions 2^-16 .. 2^16 apart and the keys' the other way.  And tiles of
+    values 2^-2 .. 2^2 apart, which they do hold.  No further from float64
+    than single precision, the sums' orders aside (its own error at 1024
+    positions is 1.1e-6)."""
+    d, lq, lk, h, hk, b = c
+    r = rng(d + lq + lk + len(form))
+    q, k, v = (r.standard_normal(s).astype(np.float32) for s in ((b, lq, h, d), (b, lk, hk, d), (b, lk, hk, d)))
+    if form == "weightless key":
+        q[..., 0], k[..., 0] = 30.0, 0.0
+        k[:, 0] = 0.0
+        k[:, 0, :, 0] = -60.0 * np.sqrt(d) / np.log2(np.e) / 30.0
+        v[:, 0] *= np.float32(2.0 ** 20)
+    elif form == "value dimensions":
+        v *= np.exp2(r.integers(-16, 17, d)).astype(np.float32)
+    elif form == "query dimensions":
+        e = np.exp2(r.integers(-16, 17, d)).astype(np.float32)
+        q, k = q * e, k / e
+    else:
+        v *= np.exp2(r.integers(-2, 3, (lk + 31) // 32)).repeat(32)[:lk, None, None].astype(np.float32)
+    got, single = attention512_case(gpu, q, k, v)
+    print(f"attention {c} {form}: {got:.3g}, single precision {single:.3g}")
+    assert got <= 1.5 * single + 1e-7
+
+
+@pytest.mark.gpu
+def test_attention512_infinities(gpu):
+    """A key of -infinity for queries above 0 has no weight and changes
+    nothing; a value of infinity makes its dimension's outputs infinite and
+    no other; a value at the end of single precision whose key has no weight
+    stays out.  As the form of single precision has it."""
+    lq = lk = 1024
+    d = 512
+    r = rng(77)
+    q, k, v = (r.standard_normal((1, n, 1, d)).astype(np.float32) for n in (lq, lk, lk))
+    q = np.abs(q)
+    k[:, 5] = -np.inf
+    v[:, 5] = np.finfo(np.float32).max
+    q_d, k_d, v_d = (dev(t, gpu).permute(0, 2, 1, 3) for t in (q, k, v))
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(d)))
+    y = unwritten((1, lq, 1, d), gpu)
+    sdhip.attention(q_d, k_d, v_d, y, scale)
+    torch.cuda.synchronize()
+    rest = np.arange(lk) != 5
+    exact, mag = orc.exact_attention(q, np.ascontiguousarray(k[:, rest]), np.ascontiguousarray(v[:, rest]), scale)
+    assert orc.metric(y.cpu().numpy(), exact, mag) <= 2 * BOUND  # single precision itself measures 1.1e-6 here
+    v[:, 7, 0, 3] = np.inf
+    v_d = dev(v, gpu).permute(0, 2, 1, 3)
+    sdhip.attention(q_d, k_d, v_d, y, scale)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert (got[..., 3] == np.inf).all()
+    assert np.isfinite(np.delete(got, 3, axis=3)).all()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("d,lq,lk,h,hk,b", [
     (40, 2081, 77, 8, 8, 2),    # workgroups of eight waves, ragged queries
