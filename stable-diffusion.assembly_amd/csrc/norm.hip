@@ -67,10 +67,16 @@ __device__ __forceinline__ double block_sum(double v, double *lds_sums) {
 }
 
 // PASS 0: the sum of x over the block's slice; PASS 1: of (x - mean)^2, each
-// difference and square in single precision (norm.cc:44-90).
+// difference and square in single precision (norm.cc:44-90); PASS 2: both in
+// double, for slices whose squares about their own mean pass single precision
+// (numbers of 9e18 and more), though those about the group's may not.
 template <int PASS>
 __device__ __forceinline__ double term(float x, float mean) {
     if (PASS == 0) return static_cast<double>(x);
+    if (PASS == 2) {
+        const double d = static_cast<double>(x) - static_cast<double>(mean);
+        return d * d;
+    }
     const float d = x - mean;
     return static_cast<double>(__fmul_rn(d, d));
 }
@@ -144,6 +150,9 @@ __global__ __launch_bounds__(kThreads) void group_stats_kernel(GroupNormArgs a) 
         sum = block_sum(slice_terms<0>(g, x, quads, 0.0f), lds_sums);
         squares = block_sum(slice_terms<1>(g, x, quads, slice_mean(sum, g.e1 - g.e0)), lds_sums);
     }
+    // The same on every thread.
+    if (!isfinite(squares))
+        squares = block_sum(slice_terms<2>(g, x, quads, slice_mean(sum, g.e1 - g.e0)), lds_sums);
     if (tid == 0) {
         a.partials[g.item * a.slices + g.slice] = sum;
         a.partials[(a.ne3 * a.groups + g.item) * a.slices + g.slice] = squares;

@@ -151,3 +151,29 @@ def test_group_norm_slices(gpu, shape, groups, offset):
     diff = np.abs(y.cpu().numpy() - want).max()
     print(f"group_norm slices {shape}/{groups}: {diff:.3g}")
     assert diff <= 1e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,groups,offset", [
+    ((1, 64, 256, 256), 32, 0),    # a slice's numbers held in registers
+    ((1, 6, 301, 211), 3, 1),      # read twice, between quads
+])
+def test_group_norm_of_great_numbers(gpu, shape, groups, offset):
+    """Numbers of +-1.5e19, whose squares about the group's mean (near 0) fit
+    single precision and, in slices that lie off it, about the slice's own mean
+    (+-7.5e18) do not.  Against float64: the difference, the scale and their
+    product round once each, outputs up to 1.2."""
+    r = rng(sum(shape))
+    n = int(np.prod(shape))
+    share = np.where(np.arange(n) // (n // groups // 2) % 2 == 0, 0.75, 0.25)  # halves of a group
+    x = np.where(r.random(n) < share, np.float32(-1.5e19), np.float32(1.5e19)).astype(np.float32).reshape(shape)
+    flat = torch.empty(n + 4, device=gpu)
+    x_d = flat[offset:offset + n].view(shape)
+    x_d.copy_(torch.from_numpy(x))
+    y = unwritten(shape, gpu)
+    sdhip.group_norm(x_d, y, groups, 1e-5)
+    torch.cuda.synchronize()
+    want = torch.nn.functional.group_norm(torch.from_numpy(x).double(), groups, eps=1e-5).numpy()
+    diff = np.abs(y.cpu().numpy() - want).max()
+    print(f"group_norm of great numbers {shape}/{groups}: {diff:.3g}")
+    assert diff <= 1e-6
