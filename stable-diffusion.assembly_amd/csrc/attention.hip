@@ -1740,10 +1740,25 @@ struct KeySplits {
 
 // Whether the keys are few enough for attention_few_kernel: their tiles fit
 // a CU's LDS, six of them at most (192 keys; beyond, the tiles' own launch is
-// repaid by the workgroups that share it).
+// repaid by the workgroups that share it).  Two head sizes have that launch
+// repaid sooner, where the queries take several rounds of waves.  Heads of 32,
+// past four tiles: 9216 queries of 8 heads and 192 keys 17.0 us by the tiles'
+// launch, 18.3 without (of one round, 4096 of 16 heads: 14.4 and 12.7).  Heads of
+// 128, whose waves have a SIMD each, where the last round is more than a fifth
+// empty: 128 keys, 9216 queries of 8 heads (2.25 rounds) 53.5 and 56.3, 1024 of 40
+// (1.25) 38.5 and 39.6; 77 keys 48.4 and 49.6, 34.4 and 33.6; full rounds 42.2 and
+// 41.9 (128 keys, 4096 of 16).
 template <int D>
 bool few_keys(const AttentionArgs &a) {
-    return ceil_div(a.lk, Few<D>::kKeys) <= Few<D>::kMostTiles;
+    const int64_t tiles = ceil_div(a.lk, Few<D>::kKeys);
+    if (tiles > Few<D>::kMostTiles) return false;
+    const int64_t waves = a.h * a.b * ceil_div(a.lq, 32), cus = compute_units();
+    if (D == 32) return tiles <= 4 || waves <= 8 * cus;
+    if (D == 128) {
+        const int64_t rounds = ceil_div(waves, 4 * cus);
+        return rounds <= (tiles == 4 ? 1 : 2) || 5 * waves >= 4 * rounds * 4 * cus;
+    }
+    return true;
 }
 
 template <int D>
@@ -1808,12 +1823,13 @@ hipError_t launch_few(const AttentionArgs &a, hipStream_t stream) {
     // Eight waves a CU share the heads' wave tiles in as few rounds as they can,
     // each about as many.  Workgroups of eight waves, or of four where those
     // would leave half the CUs without one (1024 queries of 16 heads of 80, 64
-    // workgroups of eight: 12.9 us, of four 11.9; 988 of 40 heads of 64, 160 of
-    // eight: 13.0, of four 19.1), or where a grid of eight, one dimension of
-    // under 2^32 threads, would not hold the heads.
+    // workgroups of eight: 12.9 us, of four 11.9; 4096 of 8 heads, 128 of eight:
+    // heads of 64 by 192 keys 17.1, of four 15.2, heads of 40 by 77 10.0 and 8.8;
+    // 988 of 40 heads of 64, 160 of eight: 13.0, of four 19.1), or where a grid of
+    // eight, one dimension of under 2^32 threads, would not hold the heads.
     const int64_t wave_tiles = ceil_div(a.lq, 32);
     const bool eight = F::kWaves == 8 && heads < (int64_t{1} << 23) &&
-                       2 * heads * ceil_div(wave_tiles, 8) >= compute_units();
+                       2 * heads * ceil_div(wave_tiles, 8) > compute_units();
     const int64_t waves = eight ? 8 : 4;
     const int64_t most = 8 * compute_units() / heads > waves ? 8 * compute_units() / heads : waves;
     const int64_t rounds = ceil_div(wave_tiles, most);

@@ -422,6 +422,38 @@ def test_attention_few_keys(gpu, d, lq, lk, h, hk, b):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("d,lq,lk,h,few", [
+    (32, 4096, 160, 16, True),     # five tiles of keys, one round of waves of 32 queries
+    (32, 4097, 160, 16, False),    # a wave a head more
+    (32, 4097, 128, 16, True),     # four tiles
+    (128, 1024, 128, 32, True),    # four tiles, one round of four waves a CU
+    (128, 1025, 128, 32, False),   # a second, nearly empty
+    (128, 1639, 97, 32, True),     # more than four fifths of both
+    (128, 2048, 77, 32, True),     # three tiles, two rounds
+    (128, 2049, 77, 32, False),    # a third
+    (64, 4096, 192, 8, True),      # 128 workgroups of eight waves: of four
+], ids=str)
+def test_attention_few_keys_rounds(gpu, d, lq, lk, h, few):
+    """Which calls of few keys go by the tiles' launch all the same (heads of
+    32 and 128 whose queries take several rounds of waves), on both sides of
+    each line: a sample of 300 queries within the bound of float64."""
+    sdhip.profile_reset()
+    sdhip.profile_enable(True)
+    try:
+        q, k, v, y, scale = attention_case(gpu, d, lq, lk, h, h, 1, False, seed=d + lq + lk, dist="normal")
+        names = set(sdhip.profile_collect())
+    finally:
+        sdhip.profile_enable(False)
+    assert ("attention.tiles" not in names) == few
+    queries = rng(d + lq).choice(h * lq, size=300, replace=False)
+    exact, mag = orc.exact_attention(q, k, v, scale, queries=queries)
+    err = orc.metric(y[0, queries % lq, queries // lq, :], exact, mag)
+    print(f"few keys {(d, lq, lk, h)}: {err:.3g}")
+    assert np.isfinite(y).all()
+    assert err <= BOUND
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("heads", [2 ** 22 + 1, 2 ** 23 + 1])
 def test_attention_few_keys_many_heads(gpu, heads):
     """One query and one key of more heads than workgroups of eight waves fill
