@@ -529,49 +529,92 @@ int64_t blocks_of(const WinogradArgs &a) {
 }
 
 // What a form takes on one CU, in thousands of cycles (timestamps of the three
-// kernels): a step of the input channels, and a tile's beginning and end.
+// kernels): a step of the input channels, and a tile's beginning and end; and in
+// microseconds of the whole launch, fitted as direct_faster's comment says: of
+// each round of workgroups, and of its tiles as they fill the device.
 struct Cost {
     double step, tile;
+    double us_step, us_tile, us_full_step, us_full_tile;
+};
+
+constexpr Cost kCosts[3] = {
+    {11.4, 26.0, 3.2, 12.0, 2.9, 0.0},  // Wide
+    {8.5, 14.0, 3.3, 7.8, 0.9, 0.0},    // Mid
+    {9.7, 14.0, 4.4, 7.1, 0.4, 0.8},    // Narrow
+};
+
+struct Work {
+    double cycles, us;  // of the products' launch
 };
 
 template <class S>
-double cycles_of(const WinogradArgs &a, Cost c) {
-    const int64_t rounds = ceil_div(blocks_of<S>(a), compute_units());
-    return static_cast<double>(rounds) * (static_cast<double>(ceil_div(a.ic, kChunk * S::KS)) * c.step + c.tile) + 12.0;
+Work work_of(const WinogradArgs &a, const Cost &c) {
+    const double filled = static_cast<double>(blocks_of<S>(a)) / compute_units();
+    const double rounds = static_cast<double>(ceil_div(blocks_of<S>(a), compute_units()));
+    const double steps = static_cast<double>(ceil_div(a.ic, kChunk * S::KS));
+    return {rounds * (steps * c.step + c.tile) + 12.0,
+            1.3 + rounds * (steps * c.us_step + c.us_tile) + filled * (steps * c.us_full_step + c.us_full_tile)};
 }
 
 // The form of the least cycles: 1 Wide, 2 Mid, 3 Narrow.
-int shape_of(const WinogradArgs &a, double &cycles) {
-    const double c[3] = {cycles_of<Wide>(a, {11.4, 26.0}), cycles_of<Mid>(a, {8.5, 14.0}),
-                         cycles_of<Narrow>(a, {9.7, 14.0})};
+int shape_of(const WinogradArgs &a, Work &work) {
+    const Work w[3] = {work_of<Wide>(a, kCosts[0]), work_of<Mid>(a, kCosts[1]), work_of<Narrow>(a, kCosts[2])};
     int best = 0;
     for (int i = 1; i < 3; ++i)
-        if (c[i] < c[best]) best = i;
-    cycles = c[best];
+        if (w[i].cycles < w[best].cycles) best = i;
+    work = w[best];
     return best + 1;
 }
 
-// Whether the products here take less than F(4x4)'s launches: microseconds of
-// both, fitted to measurements.  Here: the cycles at 2.3 GHz and the pass over
-// the weights.  There: the bytes of its four passes (18 an input, 22 an output,
-// 150 a kernel), its products at the rate the MFMA reaches there, its launches;
-// or, on few tiles, the small images' path, which its kernels bound.
-// Measured, here and F(4x4), us (2 images of a UNet level, 1 of the VAE's):
-//   320->320 64x64   40.4   48.8    128->128 520x768  286   595
-//   1280->640 32x32  71.7  105.1    256->256 256x256  150   217
-//   640->640 33x48   56.3   64.6    512->512 128x128  130   138
-//   1280->1280 16x16 68.2   73.9    512->512 67x117   109   107
-//   2560->1280 16x16  126    116    960->640 45x33    145   111
+// F(4x4)'s microseconds, its weights kept in the store or not: on few tiles the
+// small images' kernels, bound by the weights; else the launches; the inputs
+// and outputs (in millions), more where rows are not whole quads; the scales'
+// pass, a workgroup a channel, by single numbers where planes are not whole quads;
+// the weights' transform; the products by their rounds of workgroups and their
+// work; and what the passes between them hold past the last-level cache.
+double winograd4_us(const WinogradArgs &a, bool kept) {
+    const double kernels = static_cast<double>(a.ic * a.oc) / 1e6;
+    if (a.tiles <= 16) return kept ? 30.0 + 17.5 * kernels : 29.0 + 19.4 * kernels;
+    if (a.tiles <= 32) return kept ? 33.0 + 22.3 * kernels : 31.0 + 24.4 * kernels;
+    const double in = static_cast<double>(a.n * a.ic * a.ih * a.iw) / 1e6;
+    const double out = static_cast<double>(a.n * a.oc * a.oh * a.ow) / 1e6;
+    const double ragged = a.ow % 4 != 0 ? 1.0 : 0.0;
+    const double scales =
+        a.ih * a.iw % 4 != 0 || a.xnb1 != a.iw ? static_cast<double>(a.n * a.ih * a.iw) / 1e3 : 0.0;
+    const int64_t blocks = 36 * ceil_div(a.oc, 64) * ceil_div(a.tiles, 128);
+    const double rounds = static_cast<double>(ceil_div(blocks, 2 * compute_units()) * a.ic) / 1e3;
+    const double products = static_cast<double>(blocks * a.ic) / 1e6;
+    const double held = 144.0 * kernels + 144.0 * static_cast<double>((a.ic + a.oc) * a.tiles) / 1e6 + 4.0 * (in + out);
+    const double past = held > 200.0 ? (held - 200.0) / 100.0 : 0.0;
+    if (kept) {
+        return 20.2 + (3.3 + 0.6 * ragged) * in + (3.0 + 1.6 * ragged) * out + 1.3 * scales + 5.5 * kernels +
+               10.5 * rounds + 19.7 * products + 8.8 * past;
+    }
+    return 21.0 + (2.7 + 1.4 * ragged) * in + (2.2 + 1.5 * ragged) * out + 1.2 * scales + 34.6 * kernels +
+           3.1 * rounds + 32.0 * products + 25.0 * past;
+}
+
+// Whether the products here take less than F(4x4), by the sum of both cases, the
+// weights kept in the store and not, and by each (kept, within 2%): whichever of
+// them a call finds it takes the same path, so that its outputs do not depend on
+// the store or on a capture.  The times above were fitted to 297 shapes of the
+// UNet's and the VAE's levels, whole and ragged, with a spread of 3% for this
+// form and 4% for F(4x4).  Of those taken here none is slower by more than 2.4%
+// without the store; kept, one by 7% (12% faster without), the rest by 3.6% at
+// most.  Measured, F(4x4) and here, us, without the store and kept (images first):
+//   2 320->320 64x64   45.2 34.9   45.7 31.2   1 128->128 520x768   551  231    545  234
+//   1 640->1280 16x16  45.2 42.2   45.9 31.7   1 256->256 115x91   66.4 55.8   65.3 52.1
+//   1 1280->1280 16x16 61.2 67.7   58.9 55.7   1 256->256 196x151  99.0  112    104  108
+//   2 640->320 72x80   88.0  105   90.7 99.7   1 512->256 128x128  82.2 89.9   85.0 86.7
+//   2 1920->640 32x32   106 94.7   80.7 86.3   1 512->512 114x85    107  103    105 99.4
+//   2 2560->1280 32x32  322  210    184  191   1 128->256 104x102  40.6 41.6   42.7 38.8
 bool direct_faster(const WinogradArgs &a) {
-    double cycles = 0.0;
-    shape_of(a, cycles);
-    const double kernels = static_cast<double>(a.ic * a.oc);
-    const double in = static_cast<double>(a.n * a.ic * a.ih * a.iw), out = static_cast<double>(a.n * a.oc * a.oh * a.ow);
-    const double here = 6.0 + cycles / 2.3 + 36.0 * kernels / 4.5e6;
-    const double there =
-        a.tiles <= 32 ? 32.0 + 25.0 * kernels / 1e6
-                      : 16.0 + (18.0 * in + 22.0 * out + 150.0 * kernels) / 4.5e6 + 0.75 * 18.0 * out * a.ic / 1.1e9;
-    return here <= there;
+    Work work;
+    shape_of(a, work);
+    const double here = work.us + (a.ow % 4 != 0 ? 1.3 * static_cast<double>(a.n * a.oc * a.oh * a.ow) / 1e6 : 0.0);
+    const double weights = 3.4 + 4.9 * static_cast<double>(a.ic * a.oc) / 1e6;  // the pass over them
+    const double kept = winograd4_us(a, true), made = winograd4_us(a, false);
+    return here + weights <= made && here <= 1.02 * kept && 2.0 * here + weights <= kept + made;
 }
 
 int64_t weight_bytes(const WinogradArgs &a) { return a.ic * a.oc * 18; }
@@ -651,8 +694,8 @@ sdhip_status conv3(const WinogradArgs &a, void *work, hipStream_t stream) {
         if (kept != nullptr) store_publish(kept);
     }
     KernelScope scope("conv3x3.products", stream);
-    double cycles = 0.0;
-    const int shape = shape_of(a, cycles);
+    Work unused;
+    const int shape = shape_of(a, unused);
     const hipError_t err = shape == 1 ? launch<Wide>(p, stream) : shape == 2 ? launch<Mid>(p, stream) : launch<Narrow>(p, stream);
     return launched(err, "conv2d 3x3");
 }

@@ -499,6 +499,39 @@ def test_conv3_direct(gpu, c, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,ic,oc,h,w,direct", [
+    (2, 320, 320, 64, 64, True),     # faster either way
+    (1, 640, 1280, 16, 16, True),
+    (1, 1280, 1280, 16, 16, False),  # F(4x4)'s small images of one group of tiles: faster without the store
+    (2, 640, 320, 72, 80, False),    # slower either way
+    (1, 512, 256, 128, 128, False),
+    (2, 2560, 1280, 32, 32, True),   # half as long without the store, 3.6% longer with the weights kept
+])
+def test_conv3_line(gpu, n, ic, oc, h, w, direct):
+    """Which 3x3 convolutions go directly, on both sides of the line, and that
+    the store has no say in it: a call with an arena, one that finds its
+    weights kept and one without give the same bits."""
+    g = torch.Generator(device="cpu").manual_seed(h + w)
+    x_d = torch.randn((n, ic, h, w), generator=g).to(gpu)
+    k_d = (0.02 * torch.randn((oc, ic, 3, 3), generator=g)).half().to(gpu)
+    params = sdhip.conv_params(1, 1, 1, 1, 1, 1)
+    arena = torch.empty(160 * ic * oc + 65536, dtype=torch.uint8, device=gpu)
+    outs = []
+    try:
+        for kept in (None, arena, arena):
+            if kept is None or not outs[1:]:
+                sdhip.store_arena(kept)
+            y = unwritten((n, oc, h, w), gpu)
+            names = kernel_names(lambda: sdhip.conv2d(k_d, x_d, y, params))
+            assert ("conv3x3.products" in names) == direct
+            outs.append(y.cpu().numpy().view(np.uint32))
+        assert sdhip.store_used()[1] == 1
+    finally:
+        sdhip.store_arena(None)
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
+
+
+@pytest.mark.gpu
 def test_conv3_in_place_takes_winograd(gpu):
     """A convolution whose residual connection is written over its own inputs
     reads them all before it writes: not taken in one pass."""
