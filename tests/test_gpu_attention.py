@@ -367,6 +367,46 @@ def test_attention512_far_apart(gpu, c, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("far", [False, True])
+def test_attention512_graph_replays(gpu, far):
+    """Heads of 512 captured into a HIP graph and replayed with eager calls of
+    other numbers between the replays, in split FP16 and (values far apart) in
+    single precision: every replay equals the eager result bit for bit, and
+    the graph follows its inputs from the one to the other."""
+    g = torch.Generator().manual_seed(31)
+    q, k, v = (torch.randn((1, 1024, 1, 512), generator=g).to(gpu) for _ in range(3))
+    wide = v.clone()
+    wide[:, 7] *= 2.0 ** 20
+    scale = 512 ** -0.5
+    held = (wide if far else v).clone()
+    views = [t.permute(0, 2, 1, 3) for t in (q, k, held)]
+
+    def eager(values):
+        out = unwritten((1, 1024, 1, 512), gpu)
+        sdhip.attention(views[0], views[1], values.permute(0, 2, 1, 3), out, scale)
+        torch.cuda.synchronize()
+        return out.cpu().numpy().view(np.uint32)
+
+    want = {True: eager(wide), False: eager(v)}
+    y = torch.zeros((1, 1024, 1, 512), device=gpu)
+    graph = torch.cuda.CUDAGraph()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            work = sdhip.attention(*views, y, scale)
+    torch.cuda.current_stream().wait_stream(stream)
+    assert work is not None
+    for turn in (far, not far, far):
+        held.copy_(wide if turn else v)
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(y.cpu().numpy().view(np.uint32), want[turn])
+        assert np.array_equal(eager(v), want[False])
+
+
+@pytest.mark.gpu
 def test_attention512_infinities(gpu):
     """A key of -infinity for queries above 0 has no weight and changes
     nothing; a value of infinity makes its dimension's outputs infinite and

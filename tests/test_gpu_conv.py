@@ -499,6 +499,51 @@ def test_conv3_direct(gpu, c, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,ic,oc,h,w", [(1, 128, 128, 261, 303), (2, 320, 320, 64, 64), (2, 640, 640, 34, 34)],
+                         ids=str)
+def test_conv3_graph_replays(gpu, n, ic, oc, h, w):
+    """The direct form's three kernels captured into a HIP graph and replayed
+    with eager convolutions of other inputs between the replays: every replay
+    equals the eager result bit for bit."""
+    g = torch.Generator(device="cpu").manual_seed(h)
+    x_d = torch.randn((n, ic, h, w), generator=g).to(gpu)
+    k_d = (0.05 * torch.randn((oc, ic, 3, 3), generator=g)).half().to(gpu)
+    params = sdhip.conv_params(1, 1, 1, 1, 1, 1)
+    want = unwritten((n, oc, h, w), gpu)
+    assert "conv3x3.products" in kernel_names(lambda: sdhip.conv2d(k_d, x_d, want, params))
+    want = want.cpu().numpy().view(np.uint32)
+    y, other = torch.zeros((n, oc, h, w), device=gpu), torch.empty((n, oc, h, w), device=gpu)
+    graph = torch.cuda.CUDAGraph()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            sdhip.conv2d(k_d, x_d, y, params)
+    torch.cuda.current_stream().wait_stream(stream)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(y.cpu().numpy().view(np.uint32), want)
+        sdhip.conv2d(k_d, 2.0 * x_d, other, params)
+        torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,k", [((1, 512, 128, 128), (256, 512, 3, 3)), ((2, 640, 72, 80), (320, 640, 3, 3)),
+                                     ((2, 320, 96, 96), (96, 320, 3, 3)), ((1, 96, 512, 512), (64, 96, 3, 3))], ids=str)
+def test_winograd_large_grids(gpu, shape, k):
+    """F(4x4) at the UNet's and the VAE's sizes that do not go directly, by
+    both cores that its products choose from."""
+    errors = []
+    names = kernel_names(lambda: errors.append(sampled(gpu, shape, k, 1, 1, seed=shape[1])))
+    (err, path), = errors
+    print(f"F(4x4) {shape} {k}: sampled error {err:.3g}")
+    assert path == 4 and "winograd4.products" in names and "conv3x3.products" not in names
+    assert err <= BOUND
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,ic,oc,h,w,direct", [
     (2, 320, 320, 64, 64, True),     # faster either way
     (1, 640, 1280, 16, 16, True),

@@ -222,3 +222,65 @@ def test_kept_small_images_weight_exponents(gpu, arena, ic, oc):
     assert orc.metric(y2, exact, mag) <= 2e-5
     sdhip.forget(k_d)
     assert sdhip.store_used() == (0, 0)
+
+
+@pytest.mark.gpu
+def test_kept_direct_convolution(gpu, arena):
+    """The direct 3x3 convolution's weights, laid out for its products, kept:
+    the first call fills the entry, later calls skip the pass over them and give
+    the same outputs bit for bit as a call without a store; new weights in the
+    same memory are seen once forgotten."""
+    n, ic, oc, h_, w_ = 2, 320, 320, 64, 64
+    r = rng(9)
+    kh16, _ = weights_f16(r, (oc, ic, 3, 3))
+    k_d, x_d = dev(kh16, gpu), dev(uniform(r, (n, ic, h_, w_), 1.0), gpu)
+    sdhip.store_arena(None)
+    plain = convolve(gpu, k_d, x_d, h_, w_)
+    sdhip.store_arena(arena)
+    outs = []
+    first = kernels_of(lambda: outs.append(convolve(gpu, k_d, x_d, h_, w_)))
+    assert "conv3x3.weights" in first and "conv3x3.products" in first
+    assert sdhip.store_used() == (18 * ic * oc, 1)
+    second = kernels_of(lambda: outs.append(convolve(gpu, k_d, x_d, h_, w_)))
+    assert "conv3x3.weights" not in second and "conv3x3.products" in second
+    for y in outs:
+        assert np.array_equal(y.view(np.uint32), plain.view(np.uint32))
+    kh16, _ = weights_f16(rng(10), (oc, ic, 3, 3))
+    k_d.copy_(torch.from_numpy(kh16).to(gpu))
+    assert np.array_equal(convolve(gpu, k_d, x_d, h_, w_).view(np.uint32), plain.view(np.uint32))
+    sdhip.forget(k_d[oc - 1:])  # any byte of the weights
+    assert sdhip.store_used() == (0, 0)
+    fresh = convolve(gpu, k_d, x_d, h_, w_)
+    sdhip.store_arena(None)
+    assert np.array_equal(fresh.view(np.uint32), convolve(gpu, k_d, x_d, h_, w_).view(np.uint32))
+
+
+@pytest.mark.gpu
+def test_no_direct_convolution_entry_made_under_capture(gpu, arena):
+    """A direct convolution captured before its weights are kept lays them out
+    in its work buffer at every replay, also once an eager call has kept them."""
+    n, ic, oc, h_, w_ = 2, 320, 320, 64, 64
+    r = rng(11)
+    kh16, _ = weights_f16(r, (oc, ic, 3, 3))
+    k_d, x_d = dev(kh16, gpu), dev(uniform(r, (n, ic, h_, w_), 1.0), gpu)
+    sdhip.store_arena(None)
+    want = convolve(gpu, k_d, x_d, h_, w_)
+    sdhip.store_arena(arena)
+    y = torch.zeros((n, oc, h_, w_), device=gpu)
+    params = sdhip.conv_params(1, 1, 1, 1, 1, 1)
+    graph = torch.cuda.CUDAGraph()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            work = sdhip.conv2d(k_d, x_d, y, params)
+    torch.cuda.current_stream().wait_stream(stream)
+    torch.cuda.synchronize()
+    assert work is not None and sdhip.store_used() == (0, 0)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(y.cpu().numpy().view(np.uint32), want.view(np.uint32))
+        assert np.array_equal(convolve(gpu, k_d, x_d, h_, w_).view(np.uint32), want.view(np.uint32))
+        assert sdhip.store_used()[1] == 1
