@@ -8,10 +8,19 @@
 // MFMAs a product: 22 bits of x.  E is the workgroup's own and follows its
 // inputs as they come: it brings the greatest |x| so far into [2^13, 2^15), and
 // where a later chunk of channels passes that, the sums are rescaled (exactly)
-// and E raised.  So l is normal for every x within 2^17 of the greatest and
-// 2^-40 of that greatest off at most below, at any magnitude, and no pass over
-// the image is needed before the products.  Against 64 bits this is nearer than
-// F(4x4), whose transforms round and amplify.
+// and E raised.  So l is normal for every x within 2^15 of the greatest and
+// 2^-40 of that greatest off at most below, and no pass over the image is needed
+// before the products.  Against 64 bits this is nearer than F(4x4), whose
+// transforms round and amplify.
+//
+// An output whose kernels are small on the greatest channels needs the others'
+// own bits.  So the fetching waves also look for the least of a chunk's channels'
+// greatest |x|, and where that is below 2^-2 take the chunk two or three times,
+// 2^28 apart (store): 22 bits of each channel's greatest in the tile, the channels
+// up to 2^72 apart.  Channels 2^24 and 2^40 apart and kernels of zero on the great
+// ones, by one scale alone: 3.3e-5 and 0.45 of sum |x w| off; so, 5.1e-7.  That
+// look, wave exchanges without LDS, costs 0.3 us at 320->320, 64x64, and 2.5 at
+// 128->128, 520x768; by shuffles 1.0 and 3.8.
 //
 // Shape.  A workgroup takes tiles of kRows x 16 outputs of an image by kOc
 // output channels.  Its first waves compute, WP x WO x KS of them: WP groups of
@@ -43,6 +52,8 @@
 // positions a fragment read takes are consecutive, so fall in 16 groups of
 // banks.
 
+#include <type_traits>
+
 #include "conv3.h"
 #include "host.h"
 #include "kernels.h"
@@ -55,7 +66,9 @@ namespace {
 constexpr int kCols = 16;          // outputs of a tile's row
 constexpr int kPitch = kCols + 2;  // its inputs
 constexpr int kChunk = 32;         // input channels of a chunk
-constexpr int kMostFetch = 4;
+constexpr int kFetchWaves = kChunk / 8;
+constexpr int kLevelBits = 28;     // between the scales of a chunk's levels
+constexpr int kMostLevels = 3;
 
 template <int RW_, int NO_, int WP_, int WO_, int KS_, int FETCH>
 struct Shape {
@@ -66,23 +79,24 @@ struct Shape {
     static constexpr int kRows = RW * WP;
     static constexpr int kOc = 16 * NO * WO;
     static constexpr int kPos = (kRows + 2) * kPitch;
-    static constexpr int kItems = kPos * 4 * KS;  // (position, 8 channels)
-    static constexpr int kPer = (kItems + 64 * kFetch - 1) / (64 * kFetch);
+    static constexpr int kPosPer = (kPos + 63) / 64;  // a fetching lane's positions
+    static constexpr int kPer = KS * kPosPer;         // and its items, 8 channels of a position
     static constexpr int kPlane = kPos * 2 * kChunk;  // bytes of one part of a chunk
     static constexpr int kBuffer = KS * 2 * kPlane;
     static constexpr int kExchange = KS > 1 ? kWaves * RW * NO * 1024 : 0;
     static constexpr int kLds = 2 * kBuffer > kExchange ? 2 * kBuffer : kExchange;
     static constexpr int kOwn = RW * NO / KS;  // the tiles of 16 x 16 a wave finishes
-    static_assert(RW * NO % KS == 0 && kFetch <= kMostFetch, "whole tiles a group");
+    static_assert(RW * NO % KS == 0, "whole tiles a group");
+    static_assert(kFetch == kChunk / 8, "a fetching wave takes 8 channels of a chunk");
     static_assert(kLds + 256 <= 160 * 1024, "LDS of a CU");
 };
 
 // 256 outputs by 128 channels, eight computing waves: images of many tiles.
-using Wide = Shape<8, 2, 2, 4, 1, 4>;
+using Wide = Shape<8, 2, 2, 4, 1, kFetchWaves>;
 // 64 outputs by 160 channels, four computing waves.
-using Mid = Shape<4, 5, 1, 2, 2, 4>;
+using Mid = Shape<4, 5, 1, 2, 2, kFetchWaves>;
 // 64 outputs by 80 channels, four computing waves: few tiles.
-using Narrow = Shape<4, 5, 1, 1, 4, 4>;
+using Narrow = Shape<4, 5, 1, 1, 4, kFetchWaves>;
 
 struct Conv3Args {
     WinogradArgs a;
@@ -144,9 +158,80 @@ __device__ __forceinline__ Place place_of(const Conv3Args &p, uint32_t tile) {
 
 // What the fetching waves hand over beside the buffers.
 struct Handover {
-    float most[2][kMostFetch];  // a chunk's greatest |x|, by wave
-    int e[2];               // a buffer's exponent
+    float most[2][kFetchWaves];   // a chunk's greatest |x|, by wave,
+    float least[2][kFetchWaves];  // and the least of its channels' greatest
+    struct {
+        int e;      // a buffer's exponent,
+        int again;  // and whether the next holds what it leaves of the same chunk
+    } of[2];
 };
+
+typedef float float2v __attribute__((ext_vector_type(2)));
+
+// The lanes' values OFF (16, 32) apart: of `low`'s upper and `high`'s lower runs
+// of OFF lanes swapped, both; the greater of the two is `low`'s over each pair of
+// lanes on the lower, `high`'s on the upper.
+template <int OFF>
+__device__ __forceinline__ float2v swap_lanes(float low, float high) {
+    const uint32_t l = __builtin_bit_cast(uint32_t, low), h = __builtin_bit_cast(uint32_t, high);
+    const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(l, h, false, false)
+                             : __builtin_amdgcn_permlane16_swap(l, h, false, false);
+    const uint32_t r0 = r[0], r1 = r[1];  // a bit cast of a vector's element takes its first
+    return float2v{__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1)};
+}
+
+// The value of the lane's partner OFF (1, 2, 4, 8) apart (for 4 the eight lanes
+// mirrored: a pair has different upper halves all the same).
+template <int OFF>
+__device__ __forceinline__ float partner(float v) {
+    constexpr int kCtrl = OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : OFF == 4 ? 0x141 : 0x128;
+    const int i = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, kCtrl, 0xF, 0xF, false));
+}
+
+// Of the N values v, the lanes' own and then the greatest over pairs of lanes
+// OFF apart: halves of the values on halves of the lanes, down to one value, then
+// that value over the lanes that hold it.
+template <int OFF, int N>
+__device__ __forceinline__ void meet_lanes(float *v, int lane) {
+    constexpr int H = N > 1 ? N / 2 : 1;
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+        const float low = v[i], high = N > 1 ? v[i + H] : v[i];
+        if constexpr (OFF >= 16) {
+            const float2v r = swap_lanes<OFF>(low, high);
+            v[i] = fmaxf(r[0], r[1]);
+        } else {
+            const bool upper = (lane & OFF) != 0;
+            v[i] = fmaxf(upper ? high : low, partner<OFF>(upper ? low : high));
+        }
+    }
+    if constexpr (OFF > 1) meet_lanes<OFF / 2, H>(v, lane);
+}
+
+// The greatest (least) over the lanes that hold different values.
+template <int OFF, int N>
+__device__ __forceinline__ void range_lanes(float &most, float &least) {
+    if constexpr (OFF >= 16) {
+        const float2v m = swap_lanes<OFF>(most, most), l = swap_lanes<OFF>(least, least);
+        most = fmaxf(m[0], m[1]);
+        least = fminf(l[0], l[1]);
+    } else {
+        most = fmaxf(most, partner<OFF>(most));
+        least = fminf(least, partner<OFF>(least));
+    }
+    if constexpr (N > 2) range_lanes<OFF / 2, N / 2>(most, least);
+}
+
+// Of N values a lane, the greatest over the wave's lanes of each: the most and
+// the least positive of those (infinite if there is none).
+template <int N>
+__device__ __forceinline__ void wave_range(float (&v)[N], int lane, float &most, float &least) {
+    meet_lanes<32, N>(v, lane);
+    most = v[0];
+    least = v[0] > 0.0f ? v[0] : INFINITY;
+    range_lanes<32, N>(most, least);
+}
 
 // The fetching waves: `count` tiles from `tile` on, `stride` apart.
 template <class S>
@@ -158,23 +243,23 @@ __device__ __forceinline__ void fetch_inputs(const Conv3Args &p, uint32_t tile, 
     const int tid = static_cast<int>(threadIdx.x) - 64 * S::kWaves;
     const int lane = tid & 63, wave = tid >> 6;
     const uint32_t channel = static_cast<uint32_t>(a.xnb2) * 4;  // bytes of a channel's plane
-    // A thread's items: a position of the tile's inputs by 8 channels; their
-    // offsets in the image, past it where the position lies outside.
-    uint32_t from[S::kPer];
+    // A wave's items: channels 8 wave .. + 7 of each of the step's KS chunks at
+    // every position of the tile's inputs, 64 positions at a time; the positions'
+    // offsets in the image, past it where they lie outside.
+    uint32_t from[S::kPosPer];
     __amdgpu_buffer_rsrc_t rsrc;
     const auto locate = [&](uint32_t t) {
         const Place at = place_of<S>(p, t);
         rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.x) + static_cast<int64_t>(at.img) * a.xnb3, 0,
                                                  static_cast<int>(p.xbytes), 0x00020000);
 #pragma unroll
-        for (int u = 0; u < S::kPer; ++u) {
-            const int idx = tid + 64 * S::kFetch * u;
-            const int pos = idx % S::kPos, cg = idx / S::kPos;
+        for (int u = 0; u < S::kPosPer; ++u) {
+            const int pos = lane + 64 * u;
             const int py = pos / kPitch, px = pos - py * kPitch;
             const int iy = at.y0 + py - a.p1, ix = at.x0 + px - a.p0;
-            const bool in = idx < S::kItems && iy >= 0 && iy < a.ih && ix >= 0 && ix < a.iw;
+            const bool in = pos < S::kPos && iy >= 0 && iy < a.ih && ix >= 0 && ix < a.iw;
             from[u] = in ? static_cast<uint32_t>(iy) * static_cast<uint32_t>(a.xnb1) * 4 + static_cast<uint32_t>(ix) * 4 +
-                               8u * cg * channel
+                               8u * wave * channel
                          : kPast;
         }
     };
@@ -182,60 +267,116 @@ __device__ __forceinline__ void fetch_inputs(const Conv3Args &p, uint32_t tile, 
     const auto load = [&](int sc) {
 #pragma unroll
         for (int u = 0; u < S::kPer; ++u) {
-            const int chunk = sc * KS + (tid + 64 * S::kFetch * u) / S::kPos / 4;
-            const uint32_t at = KS > 1 && chunk >= p.chunks ? kPast : from[u];
+            const int chunk = sc * KS + u / S::kPosPer;
+            const uint32_t at = KS > 1 && chunk >= p.chunks ? kPast : from[u % S::kPosPer];
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 x[u][i] = __builtin_bit_cast(
                     float, __builtin_amdgcn_raw_buffer_load_b32(
-                               rsrc, at, static_cast<uint32_t>(sc * KS * kChunk + i) * channel, 0));
+                               rsrc, at, static_cast<uint32_t>(chunk * kChunk + i) * channel, 0));
         }
     };
+    // Of the chunk in registers: the greatest |x|, and the least of its channels'
+    // own greatest (those of zeros alone left out).
     const auto find_most = [&](int slot) {
-        float m = 0.0f;
+        float c[8 * KS];
 #pragma unroll
-        for (int u = 0; u < S::kPer; ++u)
+        for (int k = 0; k < KS; ++k)
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const float v = fabsf(x[u][i]);
-                m = fmaxf(m, v <= 3.402823466e38f ? v : 0.0f);
-            }
+                float m = 0.0f;
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-        if (lane == 0) hand.most[slot][wave] = m;
+                for (int u = 0; u < S::kPosPer; ++u) {
+                    const float v = fabsf(x[k * S::kPosPer + u][i]);
+                    m = fmaxf(m, v <= 3.402823466e38f ? v : 0.0f);
+                }
+                c[8 * k + i] = m;
+            }
+        float most, least;
+        wave_range(c, lane, most, least);
+        if (lane == 0) {
+            hand.most[slot][wave] = most;
+            hand.least[slot][wave] = least;
+        }
     };
     // The chunk's exponent: the tile's so far unless an input passes 2^15
-    // times it, then one bit of room above the chunk's.
+    // times it, then one bit of room above the chunk's.  Where a channel's
+    // greatest then lies below 2^-2, from where on l is below FP16's normal range,
+    // the chunk goes into the buffers twice: what h leaves, where it is below 2^-14
+    // and so no l of that range, follows 2^28 times as great, and once more where
+    // that channel is still below.  (A subnormal l beside it would not do: the MFMA
+    // aligns the product of a subnormal by the exponent of the least normal number,
+    // 2^-14, and cuts the sums of small products off there.)  Returns whether the
+    // chunk goes on.
     int erun = -1000;
-    const auto store = [&](int buf, bool first) {
-        float m = hand.most[buf][0];
+    int level = 0;       // of the chunk in registers
+    float reach = 0.0f;  // the least of the channels' greatest at its scale
+    const auto store = [&](int buf, int slot, bool first) {
+        float f = 1.0f;
+        if (level == 0) {
+            float m = hand.most[slot][0];
+            reach = hand.least[slot][0];
 #pragma unroll
-        for (int w = 1; w < S::kFetch; ++w) m = fmaxf(m, hand.most[buf][w]);
-        const int e = scale_exponent(m);
-        erun = first || e > erun ? e + 1 : erun;
-        const float f = ldexpf(1.0f, -erun);
-        if (tid == 0) hand.e[buf] = erun;
-#pragma unroll
-        for (int u = 0; u < S::kPer; ++u) {
-            const int idx = tid + 64 * S::kFetch * u;
-            if (idx >= S::kItems) continue;
-            half8 hi, lo;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                _Float16 h, l;
-                split_scaled(x[u][i] * f, h, l);
-                hi[i] = h;
-                lo[i] = l;
+            for (int w = 1; w < S::kFetch; ++w) {
+                m = fmaxf(m, hand.most[slot][w]);
+                reach = fminf(reach, hand.least[slot][w]);
             }
-            const int pos = idx % S::kPos, cg = idx / S::kPos;
-            char *d = lds + buf * S::kBuffer + (cg >> 2) * 2 * S::kPlane + pos * 64 + 16 * ((cg & 3) ^ ((pos >> 2) & 3));
-            *reinterpret_cast<half8 *>(d) = hi;
-            *reinterpret_cast<half8 *>(d + S::kPlane) = lo;
+            const int e = scale_exponent(m);
+            erun = first || e > erun ? e + 1 : erun;
+            f = ldexpf(1.0f, -erun);
+            reach = ldexpf(reach, -erun);
         }
+        const bool again = __builtin_amdgcn_readfirstlane(level + 1 < kMostLevels && reach < 0.25f) != 0;
+        if (tid == 0) {
+            hand.of[buf].e = erun - kLevelBits * level;
+            hand.of[buf].again = again;
+        }
+        const auto normal = [](float v) { return fabsf(v) >= 0x1p-14f ? v : 0.0f; };
+        const auto put = [&](auto keep) {
+#pragma unroll
+            for (int u = 0; u < S::kPer; ++u) {
+                const int pos = lane + 64 * (u % S::kPosPer);
+                if (pos >= S::kPos) continue;
+                half8 hi, lo;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    _Float16 h, l;
+                    const float s = x[u][i] * f;
+                    split_scaled(s, h, l);
+                    if constexpr (decltype(keep)::value) {
+                        const float hf = normal(static_cast<float>(h)), lf = normal(s - hf);
+                        const bool whole = fabsf(hf) >= 0x1p-14f && fabsf(lf) >= 0x1p-14f;
+                        h = static_cast<_Float16>(hf);
+                        l = static_cast<_Float16>(whole ? lf : 0.0f);
+                        x[u][i] = whole ? 0.0f : (s - hf) * 0x1p28f;
+                    }
+                    hi[i] = h;
+                    lo[i] = l;
+                }
+                char *d = lds + buf * S::kBuffer + u / S::kPosPer * 2 * S::kPlane + pos * 64 +
+                          16 * (wave ^ ((pos >> 2) & 3));
+                *reinterpret_cast<half8 *>(d) = hi;
+                *reinterpret_cast<half8 *>(d + S::kPlane) = lo;
+            }
+        };
+        if (again) {
+            put(std::true_type{});
+            reach *= 0x1p28f;
+            ++level;
+        } else {
+            put(std::false_type{});
+            level = 0;
+        }
+        return again;
     };
+    static_assert(kLevelBits == 28, "what a level leaves, times 2^28");
     const int chunks = count * steps;  // of all the tiles
-    int sc = 0;                        // of the chunk in registers
-    const auto advance = [&]() {
+    int sc = 0;                        // of the chunk in registers, in its tile,
+    int at = 0;                        // and of all
+    // The next buffer, and the loads of the chunk after it.
+    const auto next = [&](int buf) {
+        if (store(buf, at & 1, sc == 0)) return;
+        if (++at == chunks) return;
         if (++sc == steps) {
             sc = 0;
             tile += stride;
@@ -247,28 +388,24 @@ __device__ __forceinline__ void fetch_inputs(const Conv3Args &p, uint32_t tile, 
     load(0);
     find_most(0);
     lds_barrier();
-    store(0, true);
-    if (chunks > 1) advance();
+    next(0);
     lds_barrier();
-    int done = 0;  // chunks of the computing waves' tile
-    for (int g = 0; g < chunks; ++g) {
+    for (int g = 0;; ++g) {  // buffer g & 1 is the computing waves'
+        const bool last = at == chunks;
         if (g == 0) {  // the second chunk's greatest, beside the first's products
-            if (chunks > 1) find_most(1);
+            if (!last && level == 0) find_most(at & 1);
             lds_barrier();
         }
-        if (g + 1 < chunks) {
-            store((g + 1) & 1, sc == 0);
-            if (g + 2 < chunks) {
-                advance();
-                find_most(g & 1);
-            }
+        if (!last) {
+            next((g + 1) & 1);
+            if (at < chunks && level == 0) find_most(at & 1);
         }
-        if (KS > 1 && ++done == steps) {  // the computing waves' exchange
-            done = 0;
+        if (KS > 1 && last) {  // the computing waves' exchange: a workgroup of several groups takes one tile
             lds_barrier();
             lds_barrier();
         }
         lds_barrier();
+        if (last) break;
     }
 }
 
@@ -312,7 +449,6 @@ __device__ __forceinline__ void finish(const Conv3Args &p, const Place &at, int 
     // of its values is used: tile q is outputs x .. x + 3 of a row and channel.
     constexpr int kGroup = S::kOwn % 4 == 0 ? 4 : 5;
     static_assert(S::kOwn % kGroup == 0, "whole groups");
-    const float up = ldexpf(1.0f, erun);
     const int x = x0 + 4 * quad;
     const int xc = x + 3 < a.ow ? x : static_cast<int>(a.ow) - 4;  // of a quad, where the rows are whole quads
     const int64_t ynb[4] = {1, a.ynb1, a.ynb2, a.ynb3};
@@ -326,7 +462,8 @@ __device__ __forceinline__ void finish(const Conv3Args &p, const Place &at, int 
             const int yy = y0 + wp * RW + j / NO, oc = oc0 + 16 * (j % NO) + col;
             row[q] = yy < a.oh ? yy : static_cast<int>(a.oh) - 1;
             och[q] = oc < a.oc ? oc : static_cast<int>(a.oc) - 1;
-            t[q] = v[q0 + q] * up;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) t[q][e] = ldexpf(v[q0 + q][e], erun);
         }
         // The values of a tensor at the tiles' outputs: in one piece, or each on
         // its own.
@@ -498,10 +635,12 @@ __global__ __launch_bounds__(S::kThreads, S::kThreads / 256) void conv3_kernel(C
         for (int r = 0; r < RW; ++r)
 #pragma unroll
             for (int o = 0; o < NO; ++o) acc[r][o] = float4v{};
-        for (int sc = 0; sc < steps; ++sc, ++g) {
-            if (sc > 0) lds_barrier();
-            const int e = __builtin_amdgcn_readfirstlane(hand.e[g & 1]);
-            if (sc > 0 && e != erun) {
+        bool first = true;
+        for (int sc = 0; sc < steps; ++g) {
+            if (!first) lds_barrier();
+            const int e = __builtin_amdgcn_readfirstlane(hand.of[g & 1].e);
+            const int after = __builtin_amdgcn_readfirstlane(hand.of[g & 1].again) ? sc : sc + 1;
+            if (!first && e != erun) {
                 const float f = ldexpf(1.0f, erun - e);
 #pragma unroll
                 for (int r = 0; r < RW; ++r)
@@ -510,8 +649,10 @@ __global__ __launch_bounds__(S::kThreads, S::kThreads / 256) void conv3_kernel(C
             }
             erun = e;
             const char *buf = lds + (g & 1) * S::kBuffer + kg * 2 * S::kPlane;
-            const bool last = sc + 1 == steps;
-            chunk(buf, g == 0, oc0, sc, last ? oc_next : oc0, last ? 0 : sc + 1);
+            const bool last = after == steps;
+            chunk(buf, g == 0, oc0, sc, last ? oc_next : oc0, last ? 0 : after);
+            sc = after;
+            first = false;
         }
         finish<S>(p, at, oc0, wp, wo, kg, wave, lane, erun, acc, lds);
         lds_barrier();

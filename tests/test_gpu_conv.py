@@ -499,6 +499,39 @@ def test_conv3_direct(gpu, c, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("c", CONV3_CASES, ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("form", [18, 24, 40, 70, "ramp"], ids=str)
+def test_conv3_channels_far_apart(gpu, c, form):
+    """Some input channels 2^18 .. 2^70 times the others, and output channels
+    whose kernels on those are zero: the others' bits are held beside them.
+    `ramp` every channel on a scale of its own, 2^-35 .. 2^35, and each output
+    channel with kernels on one in sixteen.  Within the 2e-6 of test_conv3_direct
+    (both parts of an input 2^-23 of its channel's greatest off at most, the sums
+    as there)."""
+    n, ic, oc, h, w, p = c
+    g = torch.Generator(device="cpu").manual_seed(n + ic + oc + h + w + 1)
+    x = torch.randn((n, ic, h, w), generator=g)
+    k = (0.05 * torch.randn((oc, ic, 3, 3), generator=g)).half()
+    if form == "ramp":
+        x *= torch.exp2(torch.linspace(-35, 35, ic)[torch.randperm(ic, generator=g)]).view(1, ic, 1, 1)
+        k[(torch.arange(oc)[:, None] + torch.arange(ic)[None, :]) % 16 != 0] = 0
+    else:
+        great = torch.rand(ic, generator=g) < 0.05
+        great[0], great[ic - 1], great[1] = True, True, False
+        x[:, great] *= 2.0 ** form
+        k[: oc // 2, great] = 0
+    want = torch.nn.functional.conv2d(x.double(), k.double(), padding=p)
+    mag = torch.nn.functional.conv2d(x.double().abs(), k.double().abs(), padding=p)
+    x_d, k_d = x.to(gpu), k.to(gpu)
+    y = torch.full(want.shape, float("nan"), device=gpu)
+    names = kernel_names(lambda: sdhip.conv2d(k_d, x_d, y, sdhip.conv_params(1, 1, p, p, 1, 1)))
+    assert "conv3x3.products" in names
+    err = orc.metric(y.cpu().numpy(), want.numpy(), mag.numpy())
+    print(f"conv3 {c} channels apart {form}: {err:.3g}")
+    assert err <= 2e-6
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,ic,oc,h,w", [(1, 128, 128, 261, 303), (2, 320, 320, 64, 64), (2, 640, 640, 34, 34)],
                          ids=str)
 def test_conv3_graph_replays(gpu, n, ic, oc, h, w):
