@@ -113,7 +113,8 @@ const char *sdhip_last_error(void);
  * gemm_core, qgemm_core, mul_mat_panels (0: MUL_MAT by the 64 x 64 core
  * instead of the panel kernels; 2: panels of 64 x 160 only, not 64 x 64),
  * conv_panels (0:
- * 1x1 convolutions by the 64 x 64 core),
+ * 1x1 convolutions by the 64 x 64 core), conv3x3_direct (0: F(4x4,3x3) where its
+ * nine taps would be taken directly),
  * attention_generic, attention_fp32 (forms to compare, same results within
  * the bounds -- qgemm_core's bit for bit), each taking only its documented
  * values.  Returns SDHIP_ERROR
@@ -193,10 +194,14 @@ sdhip_status sdhip_mul_mat_gated(const sdhip_tensor *w, const sdhip_tensor *x, c
  * The library takes it by Winograd F(4x4,3x3) / F(2x2,3x3) where the
  * reference would (winograd_supported, four, small; winograd.cc:194-196,
  * 1204-1206, 2107-2123) and directly otherwise (conv2d_supported,
- * conv2d.cc:320-331); in the bits mode with quantize & 2, the direct
+ * conv2d.cc:320-331); of the F(4x4,3x3) calls with FP16 kernels, those of 128
+ * channels and more (inputs a multiple of 32) whose nine taps take less time as
+ * one direct product are taken so, unless the output lies over the inputs or
+ * conv3x3_direct=0 (path 4 all the same); in the bits mode with quantize & 2, the direct
  * convolution's products quantized (conv2d.cc:338-483) or F(2x2,3x3) with
  * quantized products (winograd.cc:1826-2103).  The work buffer: Winograd's
- * exponents, transformed operands and products; for a direct convolution of
+ * exponents, transformed operands and products, or the weights in the order
+ * of the direct 3x3 products, whichever is more; for a direct convolution of
  * a kernel other than 1x1 with IC KH KW a multiple of 32 (and of a 1x1 one
  * whose output has few blocks and whose K is long), its columns and the
  * partial sums of its splits of K; single-precision kernels' FP16
@@ -204,8 +209,9 @@ sdhip_status sdhip_mul_mat_gated(const sdhip_tensor *w, const sdhip_tensor *x, c
  * SDHIP_ERROR.  Replaces conv2d_* and winograd_* of ops.h:26-38. */
 int sdhip_conv2d_supported(const sdhip_tensor *kernel, const sdhip_tensor *input, const sdhip_tensor *y,
                            const int32_t op_params[6]);
-/* Which path a supported convolution takes: 0 direct, 2 Winograd F(2x2,3x3),
- * 4 Winograd F(4x4,3x3); -1 if not supported. */
+/* Which path a supported convolution takes, by the reference's rules: 0 direct,
+ * 2 Winograd F(2x2,3x3), 4 Winograd F(4x4,3x3), also where the library computes
+ * an F(4x4,3x3) call's nine taps directly; -1 if not supported. */
 int sdhip_conv2d_path(const sdhip_tensor *kernel, const sdhip_tensor *input, const sdhip_tensor *y,
                       const int32_t op_params[6]);
 size_t sdhip_conv2d_work_size(const sdhip_tensor *kernel, const sdhip_tensor *input, const sdhip_tensor *y,
@@ -227,7 +233,9 @@ sdhip_status sdhip_conv2d(const sdhip_tensor *kernel, const sdhip_tensor *input,
  * multiple of 4 from 4 to 1024, quant.cc:59-67).  The work
  * buffer: in the bits mode the quantized operands; otherwise, for
  * single-precision keys and values of the head sizes 32, 40, 64, 80, 96, 128
- * and 160, the keys and values split into FP16 parts, tile by tile, and,
+ * and 160, the keys and values split into FP16 parts, tile by tile (asked for,
+ * though not written, also where up to 192 keys are split by the workgroups
+ * that read them), and,
  * where the queries alone leave the device's CUs idle and the keys are split
  * across blocks, each split's maximum, sum and output; the same for heads of
  * more than 256 dimensions whose keys are split across blocks, and for heads

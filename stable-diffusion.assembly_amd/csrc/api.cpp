@@ -127,6 +127,7 @@ const Field kFields[] = {
     {"gemm_core", &Tuning::gemm_core, kCore},
     {"mul_mat_panels", &Tuning::mul_mat_panels, kPanels},
     {"conv_panels", &Tuning::conv_panels, kFlag},
+    {"conv3x3_direct", &Tuning::conv3x3_direct, kFlag},
     {"qgemm_core", &Tuning::qgemm_core, kFlag2},
     {"attention_generic", &Tuning::attention_generic, kFlag},
     {"attention_fp32", &Tuning::attention_fp32, kFlag},

@@ -21,6 +21,10 @@
 // ones, by one scale alone: 3.3e-5 and 0.45 of sum |x w| off; so, 5.1e-7.  That
 // look, wave exchanges without LDS, costs 0.3 us at 320->320, 64x64, and 2.5 at
 // 128->128, 520x768; by shuffles 1.0 and 3.8.
+// The second pass costs 17 of 38 us and 130 of 237; a third 15 and 110.  Not held:
+// a channel's rows further apart than its greatest's 2^-40, and kernels of FP16's
+// last bits alone (all below 2^-22; 4.4e-6 of sum |x w|, where F(4x4) scales them
+// first and has 1.8e-6).
 //
 // Shape.  A workgroup takes tiles of kRows x 16 outputs of an image by kOc
 // output channels.  Its first waves compute, WP x WO x KS of them: WP groups of
@@ -783,7 +787,7 @@ hipError_t launch(Conv3Args &p, hipStream_t stream) {
 
 bool conv3_shape(const WinogradArgs &a) {
     const Tuning &t = tuning();
-    if (a.m != 4 || a.w32 != nullptr || t.winograd_fp32 || t.gemm_core != 0 || t.gemm_tiles != 0) return false;
+    if (a.m != 4 || a.w32 != nullptr || t.winograd_fp32 || t.conv3x3_direct == 0) return false;
     if (a.ic % kChunk != 0 || a.ic < 128 || a.oc < 128) return false;
     if (a.xnb1 < a.iw || a.xnb2 < 1 || a.xnb3 < 0 || a.n < 1) return false;
     // Offsets in an image, in the weights and of blocks in 31 bits.

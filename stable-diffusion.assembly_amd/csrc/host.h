@@ -66,6 +66,9 @@ struct Tuning {
     // within the same bound.
     int mul_mat_panels = 1;
     int conv_panels = 1;
+    // This library's own: the 3x3 convolutions that are faster so directly (1)
+    // or all by F(4x4) (0), for comparison; results agree within the same bound.
+    int conv3x3_direct = 1;
     // This library's own: attention by its generic form (1) even where the
     // fast one takes the operands (0), for comparison; results agree within
     // the same bound.

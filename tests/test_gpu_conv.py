@@ -610,6 +610,32 @@ def test_conv3_line(gpu, n, ic, oc, h, w, direct):
 
 
 @pytest.mark.gpu
+def test_conv3_tuning(gpu):
+    """conv3x3_direct=0 computes by F(4x4) what goes directly, within the same
+    bound; the tuning of the products' core and blocks does not choose between
+    the two."""
+    g = torch.Generator(device="cpu").manual_seed(3)
+    x, k = torch.randn((1, 640, 16, 16), generator=g), (0.05 * torch.randn((1280, 640, 3, 3), generator=g)).half()
+    want = torch.nn.functional.conv2d(x.double(), k.double(), padding=1).numpy()
+    mag = torch.nn.functional.conv2d(x.double().abs(), k.double().abs(), padding=1).numpy()
+    x_d, k_d = x.to(gpu), k.to(gpu)
+    outs = {}
+    for tuning in ("", "gemm_core=3,gemm_tiles=22", "gemm_core=1", "conv3x3_direct=0"):
+        y = unwritten((1, 1280, 16, 16), gpu)
+        sdhip.set_tuning(tuning)
+        try:
+            names = kernel_names(lambda: sdhip.conv2d(k_d, x_d, y, sdhip.conv_params(1, 1, 1, 1, 1, 1)))
+        finally:
+            sdhip.set_tuning("")
+        assert ("conv3x3.products" in names) == (tuning != "conv3x3_direct=0"), tuning
+        assert ("winograd4.products" in names) == (tuning == "conv3x3_direct=0"), tuning
+        outs[tuning] = y.cpu().numpy()
+        assert orc.metric(outs[tuning], want, mag) <= BOUND, tuning
+    for tuning in ("gemm_core=3,gemm_tiles=22", "gemm_core=1"):
+        assert np.array_equal(outs[tuning].view(np.uint32), outs[""].view(np.uint32))
+
+
+@pytest.mark.gpu
 def test_conv3_in_place_takes_winograd(gpu):
     """A convolution whose residual connection is written over its own inputs
     reads them all before it writes: not taken in one pass."""
