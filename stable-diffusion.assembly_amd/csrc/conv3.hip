@@ -19,8 +19,8 @@
 // 2^28 apart (store): 22 bits of each channel's greatest in the tile, the channels
 // up to 2^72 apart.  Channels 2^24 and 2^40 apart and kernels of zero on the great
 // ones, by one scale alone: 3.3e-5 and 0.45 of sum |x w| off; so, 5.1e-7.  That
-// look, wave exchanges without LDS, costs 0.3 us at 320->320, 64x64, and 2.5 at
-// 128->128, 520x768; by shuffles 1.0 and 3.8.
+// look, over the lanes by exchanges without LDS and on the numbers' bits, costs 0.3
+// us at 320->320, 64x64, and 1 .. 2 at 128->128, 520x768; by shuffles 1.0 and 3.8.
 // The second pass costs 17 of 38 us and 130 of 237; a third 15 and 110.  Not held:
 // a channel's rows further apart than its greatest's 2^-40, and kernels of FP16's
 // last bits alone (all below 2^-22; 4.4e-6 of sum |x w|, where F(4x4) scales them
@@ -170,71 +170,69 @@ struct Handover {
     } of[2];
 };
 
-typedef float float2v __attribute__((ext_vector_type(2)));
+// Magnitudes are compared as the bits of |x|, whose order is theirs (infinities
+// and NaN above all others, from kInfinite on).
+constexpr uint32_t kInfinite = 0x7f800000u;
+
+__device__ __forceinline__ uint32_t greater(uint32_t a, uint32_t b) { return a > b ? a : b; }
 
 // The lanes' values OFF (16, 32) apart: of `low`'s upper and `high`'s lower runs
-// of OFF lanes swapped, both; the greater of the two is `low`'s over each pair of
-// lanes on the lower, `high`'s on the upper.
+// of OFF lanes swapped, the greater of both: `low`'s over each pair of lanes on
+// the lower, `high`'s on the upper.
 template <int OFF>
-__device__ __forceinline__ float2v swap_lanes(float low, float high) {
-    const uint32_t l = __builtin_bit_cast(uint32_t, low), h = __builtin_bit_cast(uint32_t, high);
-    const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(l, h, false, false)
-                             : __builtin_amdgcn_permlane16_swap(l, h, false, false);
-    const uint32_t r0 = r[0], r1 = r[1];  // a bit cast of a vector's element takes its first
-    return float2v{__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1)};
+__device__ __forceinline__ uint32_t swapped_greater(uint32_t low, uint32_t high) {
+    const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(low, high, false, false)
+                             : __builtin_amdgcn_permlane16_swap(low, high, false, false);
+    return greater(r[0], r[1]);
 }
 
 // The value of the lane's partner OFF (1, 2, 4, 8) apart (for 4 the eight lanes
 // mirrored: a pair has different upper halves all the same).
 template <int OFF>
-__device__ __forceinline__ float partner(float v) {
+__device__ __forceinline__ uint32_t partner(uint32_t v) {
     constexpr int kCtrl = OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : OFF == 4 ? 0x141 : 0x128;
-    const int i = __builtin_bit_cast(int, v);
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, kCtrl, 0xF, 0xF, false));
+    const int i = static_cast<int>(v);
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(i, i, kCtrl, 0xF, 0xF, false));
 }
 
 // Of the N values v, the lanes' own and then the greatest over pairs of lanes
 // OFF apart: halves of the values on halves of the lanes, down to one value, then
 // that value over the lanes that hold it.
 template <int OFF, int N>
-__device__ __forceinline__ void meet_lanes(float *v, int lane) {
+__device__ __forceinline__ void meet_lanes(uint32_t *v, int lane) {
     constexpr int H = N > 1 ? N / 2 : 1;
 #pragma unroll
     for (int i = 0; i < H; ++i) {
-        const float low = v[i], high = N > 1 ? v[i + H] : v[i];
+        const uint32_t low = v[i], high = N > 1 ? v[i + H] : v[i];
         if constexpr (OFF >= 16) {
-            const float2v r = swap_lanes<OFF>(low, high);
-            v[i] = fmaxf(r[0], r[1]);
+            v[i] = swapped_greater<OFF>(low, high);
         } else {
             const bool upper = (lane & OFF) != 0;
-            v[i] = fmaxf(upper ? high : low, partner<OFF>(upper ? low : high));
+            v[i] = greater(upper ? high : low, partner<OFF>(upper ? low : high));
         }
     }
     if constexpr (OFF > 1) meet_lanes<OFF / 2, H>(v, lane);
 }
 
-// The greatest (least) over the lanes that hold different values.
+// The greatest over the lanes that hold different ones of N values.
 template <int OFF, int N>
-__device__ __forceinline__ void range_lanes(float &most, float &least) {
+__device__ __forceinline__ uint32_t over_lanes(uint32_t v) {
     if constexpr (OFF >= 16) {
-        const float2v m = swap_lanes<OFF>(most, most), l = swap_lanes<OFF>(least, least);
-        most = fmaxf(m[0], m[1]);
-        least = fminf(l[0], l[1]);
+        v = swapped_greater<OFF>(v, v);
     } else {
-        most = fmaxf(most, partner<OFF>(most));
-        least = fminf(least, partner<OFF>(least));
+        v = greater(v, partner<OFF>(v));
     }
-    if constexpr (N > 2) range_lanes<OFF / 2, N / 2>(most, least);
+    if constexpr (N > 2) v = over_lanes<OFF / 2, N / 2>(v);
+    return v;
 }
 
-// Of N values a lane, the greatest over the wave's lanes of each: the most and
-// the least positive of those (infinite if there is none).
+// Of N magnitudes a lane, the greatest over the wave's lanes of each: the most and
+// the least positive of those (kInfinite if there is none).
 template <int N>
-__device__ __forceinline__ void wave_range(float (&v)[N], int lane, float &most, float &least) {
+__device__ __forceinline__ void wave_range(uint32_t (&v)[N], int lane, uint32_t &most, uint32_t &least) {
     meet_lanes<32, N>(v, lane);
-    most = v[0];
-    least = v[0] > 0.0f ? v[0] : INFINITY;
-    range_lanes<32, N>(most, least);
+    most = over_lanes<32, N>(v[0]);
+    least = ~over_lanes<32, N>(~(v[0] != 0 ? v[0] : kInfinite));
 }
 
 // The fetching waves: `count` tiles from `tile` on, `stride` apart.
@@ -281,26 +279,45 @@ __device__ __forceinline__ void fetch_inputs(const Conv3Args &p, uint32_t tile, 
         }
     };
     // Of the chunk in registers: the greatest |x|, and the least of its channels'
-    // own greatest (those of zeros alone left out).
+    // own greatest (those of zeros alone left out); of its finite numbers, where
+    // some are not.
     const auto find_most = [&](int slot) {
-        float c[8 * KS];
+        uint32_t c[8 * KS];
+        uint32_t most, least;
 #pragma unroll
         for (int k = 0; k < KS; ++k)
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                float m = 0.0f;
+                // The greatest of the positive and of the negative numbers: two
+                // operations for two numbers, signed and unsigned.
+                int32_t above = 0;
+                uint32_t below = 0;
 #pragma unroll
                 for (int u = 0; u < S::kPosPer; ++u) {
-                    const float v = fabsf(x[k * S::kPosPer + u][i]);
-                    m = fmaxf(m, v <= 3.402823466e38f ? v : 0.0f);
+                    const uint32_t bits = __builtin_bit_cast(uint32_t, x[k * S::kPosPer + u][i]);
+                    above = static_cast<int32_t>(bits) > above ? static_cast<int32_t>(bits) : above;
+                    below = greater(below, bits);
                 }
-                c[8 * k + i] = m;
+                c[8 * k + i] = greater(static_cast<uint32_t>(above), below & 0x7fffffffu);
             }
-        float most, least;
         wave_range(c, lane, most, least);
+        if (__builtin_amdgcn_readfirstlane(most) >= kInfinite) {
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    c[8 * k + i] = 0;
+#pragma unroll
+                    for (int u = 0; u < S::kPosPer; ++u) {
+                        const uint32_t m = __builtin_bit_cast(uint32_t, x[k * S::kPosPer + u][i]) & 0x7fffffffu;
+                        c[8 * k + i] = greater(c[8 * k + i], m < kInfinite ? m : 0);
+                    }
+                }
+            wave_range(c, lane, most, least);
+        }
         if (lane == 0) {
-            hand.most[slot][wave] = most;
-            hand.least[slot][wave] = least;
+            hand.most[slot][wave] = __builtin_bit_cast(float, most);
+            hand.least[slot][wave] = __builtin_bit_cast(float, least);
         }
     };
     // The chunk's exponent: the tile's so far unless an input passes 2^15
