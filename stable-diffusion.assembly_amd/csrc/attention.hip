@@ -1802,6 +1802,10 @@ size_t split_tiles_bytes(const AttentionArgs &a) {
     return static_cast<size_t>(a.b * a.hk) * static_cast<size_t>(ceil_div(a.lk, SplitShape<D>::kKeys)) * S::kRecord;
 }
 
+// The size asked for is the tiles' also where the keys are few and
+// attention_few_kernel takes no buffer: which of the two a call takes depends on
+// its queries (few_keys), and a buffer sized for one call of a program serves its
+// others.
 template <int D>
 size_t split_work(const AttentionArgs &a) {
     const KeySplits ks = key_splits<D>(a);

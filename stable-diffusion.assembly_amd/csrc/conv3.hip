@@ -45,16 +45,18 @@
 // What bounds it (timestamps of the waves, cycles).  A chunk of the 256 x 128
 // form is 9216 cycles of MFMA on each SIMD and takes 11400, the MFMA's rate at
 // 81%; a tile's end, 25000, is HBM's, every CU reading its residual and writing
-// its outputs at once: 128->128 at 520x768 with a residual 595 -> 278 us, of
-// which the bytes (614 MB, once each) are 119 at a copy's rate.  The 64 x 160
+// its outputs at once: 128->128 at 520x768 with a residual 595 -> 287 us (a call
+// among others on new inputs each, the weights not kept, as all the times here),
+// of which the bytes (614 MB, once each) are 119 at a copy's rate.  The 64 x 160
 // form has one computing wave on a SIMD, 8300 cycles a pair of chunks of 5760 of
 // MFMA, a start of 10000 and an end of 13500: 320->320 at 64x64, two images,
-// 47.0 -> 35.8 us.  Not faster: two workgroups of 128 x 128 a CU (332 us at
+// 47.6 -> 36.4 us.  Not faster: two workgroups of 128 x 128 a CU (332 us at
 // 520x768), the residual's lines read ahead by the fetching waves (298), stores
 // past the caches (293), raised priority for either kind of wave.
-// 16-byte piece p of a position's 64 bytes lies at p ^ (position / 4 % 4): the 16
-// positions a fragment read takes are consecutive, so fall in 16 groups of
-// banks.
+// 16-byte piece p of a position's 64 bytes lies at p ^ (position / 4 % 4), so that
+// the 16 consecutive positions of a fragment lie in 16 groups of banks for each
+// piece; the counter still has 3.3 conflicts an LDS instruction in the 64 x 160
+// form (reads, the fetching waves' writes and the exchange together).
 
 #include <type_traits>
 
@@ -763,7 +765,7 @@ double winograd4_us(const WinogradArgs &a, bool kept) {
 // UNet's and the VAE's levels, whole and ragged, with a spread of 3% for this
 // form and 4% for F(4x4).  Of those taken here none is slower by more than 2.4%
 // without the store; kept, one by 7% (12% faster without), the rest by 3.6% at
-// most.  Measured, F(4x4) and here, us, without the store and kept (images first):
+// most (the look at the channels, later, adds 0.5 .. 1.5% to this form).  Measured, F(4x4) and here, us, without the store and kept (images first):
 //   2 320->320 64x64   45.2 34.9   45.7 31.2   1 128->128 520x768   551  231    545  234
 //   1 640->1280 16x16  45.2 42.2   45.9 31.7   1 256->256 115x91   66.4 55.8   65.3 52.1
 //   1 1280->1280 16x16 61.2 67.7   58.9 55.7   1 256->256 196x151  99.0  112    104  108
