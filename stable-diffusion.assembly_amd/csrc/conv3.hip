@@ -19,9 +19,12 @@
 // 2^28 apart (store): 22 bits of each channel's greatest in the tile, the channels
 // up to 2^72 apart.  Channels 2^24 and 2^40 apart and kernels of zero on the great
 // ones, by one scale alone: 3.3e-5 and 0.45 of sum |x w| off; so, 5.1e-7.  That
-// look, over the lanes by exchanges without LDS and on the numbers' bits, costs 0.3
-// us at 320->320, 64x64, and 1 .. 2 at 128->128, 520x768; by shuffles 1.0 and 3.8.
-// The second pass costs 17 of 38 us and 130 of 237; a third 15 and 110.  Not held:
+// look, two numbers an operation and over the lanes without LDS, costs nothing in
+// the forms of few tiles and 1 .. 2% of the 256 x 128 one, whose code it takes past
+// the instruction cache (by shuffles 1 .. 3%; the second pass's code in a loop that
+// is not unrolled 1% less there and twice the time below).  The second pass costs 16
+// of 38 us at 320->320, 64x64, and 115 of 227 at 128->128, 520x768; a third 15 and
+// 115.  Not held:
 // a channel's rows further apart than its greatest's 2^-40, and kernels of FP16's
 // last bits alone (all below 2^-22; 4.4e-6 of sum |x w|, where F(4x4) scales them
 // first and has 1.8e-6).
@@ -164,9 +167,11 @@ __device__ __forceinline__ Place place_of(const Conv3Args &p, uint32_t tile) {
 
 // What the fetching waves hand over beside the buffers.
 struct Handover {
-    float most[2][kFetchWaves];   // a chunk's greatest |x|, by wave,
-    float least[2][kFetchWaves];  // and the least of its channels' greatest
-    struct {
+    struct alignas(8) {
+        float most;   // a chunk's greatest |x|, by wave,
+        float least;  // and the least of its channels' greatest
+    } range[2][kFetchWaves];
+    struct alignas(8) {
         int e;      // a buffer's exponent,
         int again;  // and whether the next holds what it leaves of the same chunk
     } of[2];
@@ -290,20 +295,16 @@ __device__ __forceinline__ void fetch_inputs(const Conv3Args &p, uint32_t tile, 
         for (int k = 0; k < KS; ++k)
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                // The greatest of the positive and of the negative numbers: two
-                // operations for two numbers, signed and unsigned.
-                int32_t above = 0;
-                uint32_t below = 0;
+                // One operation for two numbers: |.| is part of it, and a NaN
+                // goes through.
+                float m = fabsf(x[k * S::kPosPer][i]);
 #pragma unroll
-                for (int u = 0; u < S::kPosPer; ++u) {
-                    const uint32_t bits = __builtin_bit_cast(uint32_t, x[k * S::kPosPer + u][i]);
-                    above = static_cast<int32_t>(bits) > above ? static_cast<int32_t>(bits) : above;
-                    below = greater(below, bits);
-                }
-                c[8 * k + i] = greater(static_cast<uint32_t>(above), below & 0x7fffffffu);
+                for (int u = 1; u < S::kPosPer; ++u)
+                    m = __builtin_elementwise_maximum(m, fabsf(x[k * S::kPosPer + u][i]));
+                c[8 * k + i] = __builtin_bit_cast(uint32_t, m);
             }
         wave_range(c, lane, most, least);
-        if (__builtin_amdgcn_readfirstlane(most) >= kInfinite) {
+        if (__builtin_expect(__builtin_amdgcn_readfirstlane(most) >= kInfinite, 0)) {
 #pragma unroll
             for (int k = 0; k < KS; ++k)
 #pragma unroll
@@ -318,8 +319,8 @@ __device__ __forceinline__ void fetch_inputs(const Conv3Args &p, uint32_t tile, 
             wave_range(c, lane, most, least);
         }
         if (lane == 0) {
-            hand.most[slot][wave] = __builtin_bit_cast(float, most);
-            hand.least[slot][wave] = __builtin_bit_cast(float, least);
+            hand.range[slot][wave].most = __builtin_bit_cast(float, most);
+            hand.range[slot][wave].least = __builtin_bit_cast(float, least);
         }
     };
     // The chunk's exponent: the tile's so far unless an input passes 2^15
@@ -337,12 +338,12 @@ __device__ __forceinline__ void fetch_inputs(const Conv3Args &p, uint32_t tile, 
     const auto store = [&](int buf, int slot, bool first) {
         float f = 1.0f;
         if (level == 0) {
-            float m = hand.most[slot][0];
-            reach = hand.least[slot][0];
+            float m = hand.range[slot][0].most;
+            reach = hand.range[slot][0].least;
 #pragma unroll
             for (int w = 1; w < S::kFetch; ++w) {
-                m = fmaxf(m, hand.most[slot][w]);
-                reach = fminf(reach, hand.least[slot][w]);
+                m = fmaxf(m, hand.range[slot][w].most);
+                reach = fminf(reach, hand.range[slot][w].least);
             }
             const int e = scale_exponent(m);
             erun = first || e > erun ? e + 1 : erun;
@@ -382,7 +383,7 @@ __device__ __forceinline__ void fetch_inputs(const Conv3Args &p, uint32_t tile, 
                 *reinterpret_cast<half8 *>(d + S::kPlane) = lo;
             }
         };
-        if (again) {
+        if (__builtin_expect(again, 0)) {
             put(std::true_type{});
             reach *= 0x1p28f;
             ++level;
@@ -765,7 +766,7 @@ double winograd4_us(const WinogradArgs &a, bool kept) {
 // UNet's and the VAE's levels, whole and ragged, with a spread of 3% for this
 // form and 4% for F(4x4).  Of those taken here none is slower by more than 2.4%
 // without the store; kept, one by 7% (12% faster without), the rest by 3.6% at
-// most (the look at the channels, later, adds 0.5 .. 1.5% to this form).  Measured, F(4x4) and here, us, without the store and kept (images first):
+// most (the look at the channels, later, adds 0 .. 2% to this form).  Measured, F(4x4) and here, us, without the store and kept (images first):
 //   2 320->320 64x64   45.2 34.9   45.7 31.2   1 128->128 520x768   551  231    545  234
 //   1 640->1280 16x16  45.2 42.2   45.9 31.7   1 256->256 115x91   66.4 55.8   65.3 52.1
 //   1 1280->1280 16x16 61.2 67.7   58.9 55.7   1 256->256 196x151  99.0  112    104  108
