@@ -48,17 +48,17 @@
 // What bounds it (timestamps of the waves, cycles).  A chunk of the 256 x 128
 // form is 9216 cycles of MFMA on each SIMD and takes 11400, the MFMA's rate at
 // 81%; a tile's end, 25000, is HBM's, every CU reading its residual and writing
-// its outputs at once: 128->128 at 520x768 with a residual 595 -> 287 us (a call
+// its outputs at once: 128->128 at 520x768 with a residual 595 -> 285 us (a call
 // among others on new inputs each, the weights not kept, as all the times here),
 // of which the bytes (614 MB, once each) are 119 at a copy's rate.  The 64 x 160
 // form has one computing wave on a SIMD, 8300 cycles a pair of chunks of 5760 of
 // MFMA, a start of 10000 and an end of 13500: 320->320 at 64x64, two images,
-// 47.6 -> 36.4 us.  Not faster: two workgroups of 128 x 128 a CU (332 us at
+// 47.6 -> 35.4 us.  Not faster: two workgroups of 128 x 128 a CU (332 us at
 // 520x768), the residual's lines read ahead by the fetching waves (298), stores
 // past the caches (293), raised priority for either kind of wave.
 // 16-byte piece p of a position's 64 bytes lies at p ^ (position / 4 % 4), so that
 // the 16 consecutive positions of a fragment lie in 16 groups of banks for each
-// piece; the counter still has 3.3 conflicts an LDS instruction in the 64 x 160
+// piece; the counter still has 3.4 conflicts an LDS instruction in the 64 x 160
 // form (reads, the fetching waves' writes and the exchange together).
 
 #include <type_traits>
