@@ -532,6 +532,33 @@ def test_conv3_channels_far_apart(gpu, c, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("c", CONV3_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_conv3_not_finite(gpu, c):
+    """Infinities and NaN in a few inputs, great channels 2^24 times the others
+    beside them: the outputs they reach are not finite, and all others are within
+    the 2e-6 of test_conv3_channels_far_apart."""
+    n, ic, oc, h, w, p = c
+    g = torch.Generator(device="cpu").manual_seed(n + ic + oc + h + w + 2)
+    x = torch.randn((n, ic, h, w), generator=g)
+    k = (0.05 * torch.randn((oc, ic, 3, 3), generator=g)).half()
+    x[:, 5] *= 2.0 ** 24
+    k[: oc // 2, 5] = 0
+    for i, (ch, y, z) in enumerate(((0, 3, 7), (5, 20, 11), (ic - 1, h - 1, w - 1))):
+        x[i % n, ch, y, z] = (float("inf"), float("nan"), -float("inf"))[i]
+    want = torch.nn.functional.conv2d(x.double(), k.double(), padding=p)
+    mag = torch.nn.functional.conv2d(x.double().abs(), k.double().abs(), padding=p)
+    reached = torch.nn.functional.conv2d((~torch.isfinite(x)).float(), torch.ones((1, ic, 3, 3)), padding=p) > 0
+    reached = reached.expand(want.shape).numpy()
+    x_d, k_d = x.to(gpu), k.to(gpu)
+    y = torch.zeros(want.shape, device=gpu)
+    names = kernel_names(lambda: sdhip.conv2d(k_d, x_d, y, sdhip.conv_params(1, 1, p, p, 1, 1)))
+    assert "conv3x3.products" in names
+    got = y.cpu().numpy()
+    assert not np.isfinite(got[reached]).any() and np.isfinite(got[~reached]).all()
+    assert orc.metric(got[~reached], want.numpy()[~reached], mag.numpy()[~reached]) <= 2e-6
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,ic,oc,h,w", [(1, 128, 128, 261, 303), (2, 320, 320, 64, 64), (2, 640, 640, 34, 34)],
                          ids=str)
 def test_conv3_graph_replays(gpu, n, ic, oc, h, w):
